@@ -33,7 +33,8 @@ __global__ void k_q8_mma(const KtGemvArgs, const KtGroupedArgs, const int8_t*, c
 template <int SRC> __global__ void k_tern_pack(const uint8_t*, const uint16_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_q8_pack(const uint8_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_tern_pack_ptq1(const uint8_t*, int, int, int, int, uint32_t*, uint16_t*);
-extern "C" __global__ void k_quant_tern(const float*, int, int, int, int8_t*, int, float*, int*);
+template <bool HP> __global__ void k_quant_tern(const float*, int, int, int, int8_t*, int, float*, int*);
+template <int NR> __global__ void k_quant_row(const float*, int, int, int8_t*, int, float*, int*);
 extern "C" __global__ void k_quant_q8(const float*, int, int, int, int8_t*, int, float*, int);
 extern "C" __global__ void k_tern_sum(const float*, float*, int, int, int);
 template <bool DBG, bool RS>
@@ -496,8 +497,28 @@ int kt_quant_q8(const float* X, int ldx, int M, int C, int per_row, int8_t* XQ, 
   if(M == 0) return 0;
   if(!X || !XQ || !XS || !XA || M < 0 || C <= 0 || C % 128 || ldx < C || ldq < C || ldx % 2 || ldq % 16
      || !kt_al(X, 8) || !kt_al(XQ, 16) || per_row < 0 || per_row > 2) return KT_INVALID;
-  KT_LAUNCH(k_quant_tern, dim3(M), dim3(256), 0, kt_stream(stream), X, ldx, C, per_row, XQ, ldq,
-                     XS, (int*)XA);
+  const int NG = C / 128;
+  hipStream_t s = kt_stream(stream);
+  if(per_row == 1){
+    const int nr = (NG + 7) / 8;                             /* groups a wave */
+    for(int m0 = 0; m0 < M; m0 += 1 << 22){                  /* a launch takes fewer than 2^32 threads */
+      const dim3 grid(M - m0 < (1 << 22) ? M - m0 : 1 << 22);
+      const float* x = X + (long long)m0 * ldx;
+      int8_t* q = XQ + (long long)m0 * ldq;
+      float* xs = XS + (long long)m0 * NG;
+      int* xa = (int*)XA + (long long)m0 * NG;
+#define KT_QR(NR) KT_LAUNCH((k_quant_row<NR>), grid, dim3(512), 0, s, x, ldx, C, q, ldq, xs, xa)
+      if(nr <= 4) KT_QR(4); else if(nr <= 8) KT_QR(8); else if(nr <= 16) KT_QR(16); else if(nr <= 32) KT_QR(32);
+      else KT_QR(0);
+#undef KT_QR
+    }
+    return 0;
+  }
+  /* chunks of a row: one group a wave while the rows are few, down to one block a row from 4096 rows (16 blocks of 4
+     waves a CU) */
+  const int most = (NG + 3) / 4, want = 4096 / M > 1 ? 4096 / M : 1, nch = want < most ? want : most;
+  if(per_row == 2) KT_LAUNCH((k_quant_tern<true>), dim3(M * nch), dim3(256), 0, s, X, ldx, C, nch, XQ, ldq, XS, (int*)XA);
+  else KT_LAUNCH((k_quant_tern<false>), dim3(M * nch), dim3(256), 0, s, X, ldx, C, nch, XQ, ldq, XS, (int*)XA);
   return 0;
 }
 

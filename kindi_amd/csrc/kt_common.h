@@ -161,3 +161,11 @@ template <int X> __device__ __forceinline__ double kf_xord(double v){
   const int lo = kf_xor<X>((int)b), hi = kf_xor<X>((int)(b >> 32));
   return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
+__device__ __forceinline__ float kf_wave_max(float m){   /* every lane: the wave's maximum */
+  m = fmaxf(m, kf_xorf<1>(m)); m = fmaxf(m, kf_xorf<2>(m)); m = fmaxf(m, kf_xorf<4>(m));
+  m = fmaxf(m, kf_xorf<8>(m)); m = fmaxf(m, kf_xorf<16>(m)); return fmaxf(m, kf_xorf<32>(m));
+}
+__device__ __forceinline__ int kf_wave_sum(int v){
+  v += kf_xor<1>(v); v += kf_xor<2>(v); v += kf_xor<4>(v); v += kf_xor<8>(v); v += kf_xor<16>(v);
+  return v + kf_xor<32>(v);
+}

@@ -31,15 +31,6 @@
 template <int X> __device__ __forceinline__ float kf_bfly(float v, unsigned neg){
   return __int_as_float(__float_as_int(v) ^ neg) + kf_xorf<X>(v);
 }
-__device__ __forceinline__ float kf_wave_max(float m){   /* every lane: the wave's maximum */
-  m = fmaxf(m, kf_xorf<1>(m)); m = fmaxf(m, kf_xorf<2>(m)); m = fmaxf(m, kf_xorf<4>(m));
-  m = fmaxf(m, kf_xorf<8>(m)); m = fmaxf(m, kf_xorf<16>(m)); return fmaxf(m, kf_xorf<32>(m));
-}
-__device__ __forceinline__ int kf_wave_sum(int v){
-  v += kf_xor<1>(v); v += kf_xor<2>(v); v += kf_xor<4>(v); v += kf_xor<8>(v); v += kf_xor<16>(v);
-  return v + kf_xor<32>(v);
-}
-
 template <int NM>
 __device__ __forceinline__ void kf_fwht(float* v, float* sm, int j, int HB){
   const int l = j & 63;
