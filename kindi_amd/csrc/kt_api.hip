@@ -79,6 +79,7 @@ size_t kt_moe1_down_lds(int k, int KS);
 #ifndef KT_PAIR_WAVES
 #define KT_PAIR_WAVES 6144             /* one-token grids of more waves take two row groups a block (k_gemv_pair) */
 #endif
+#define KT_RT_BLOCK 512                /* k_moe_route's threads (kt_moe.hip KT_RT_WAVES waves) */
 #define KT_RS_BLOCKS 1024              /* per-row prefill on small blocks while the 128 x 128 grid has fewer blocks */
 
 static inline hipStream_t kt_stream(void* s){ return (hipStream_t)s; }
@@ -327,7 +328,7 @@ static int kt_moe_decode_run(const void* const* Wup, const void* const* Wdown, i
     return 0;
   }
   /* 1: router, top-k, lists */
-  KT_LAUNCH(k_moe_route, dim3(1), dim3(256), 0, s, logits, M, E, k, rt, ids, gw, cnt, off, xrow, where, act, nact,
+  KT_LAUNCH(k_moe_route, dim3(1), dim3(KT_RT_BLOCK), 0, s, logits, M, E, k, rt, ids, gw, cnt, off, xrow, where, act, nact,
                      (const float*)nullptr, 0, 0, (int8_t*)nullptr, 0, (float*)nullptr, 0);
   const int n = M * k;
   /* 2: up = W_e x[xrow[p]] per entry, x quantized in the staging */
@@ -747,7 +748,7 @@ int kt_moe_route_r(const float* logits, int M, int E, int k, int score, const fl
   if(!logits || !ids || !gw || !cnt || !off || !xrow || !where || !act || !nact || M < 0 || E <= 0 || E > 1024 ||
      k <= 0 || k > 16 || k > E || M > 64 || (long long)M * k > 64) return KT_INVALID;
   if(x && (H <= 0 || H % 32 || ldx < H || !Q || ldq < H || !D || ldd < H / 32)) return KT_INVALID;
-  KT_LAUNCH(k_moe_route, dim3(1), dim3(256), 0, kt_stream(stream), logits, M, E, k, rt, ids, gw, cnt, off, xrow,
+  KT_LAUNCH(k_moe_route, dim3(1), dim3(KT_RT_BLOCK), 0, kt_stream(stream), logits, M, E, k, rt, ids, gw, cnt, off, xrow,
             where, act, nact, x, ldx, H, Q, ldq, D, ldd);
   return 0;
 }

@@ -8,7 +8,7 @@
                     (stable), so the lists are deterministic.
    (the grouped product itself, per active expert and its token list, is the decode product k_gemv_flat in its
    grouped mode, kt_gemv.h: the dense q8_0 product's lanes, arithmetic and summation tree; output row = entry)
-     k_moe_route    k_moe_topk and k_moe_sort in one launch by one wave, for up to 64 entries.
+     k_moe_route    k_moe_topk and k_moe_sort in one launch of one block, for up to 64 entries.
      k_moe_combine  x[t] += sum_j fmaf(gw[t k + j], yd[where[t k + j]], .) (+ ysh[t]); x and ysh rows ldx apart.
 */
 #include "kt_common.h"
@@ -114,35 +114,45 @@ extern "C" __global__ void __launch_bounds__(1024) k_moe_sort(const int* __restr
   kt_moe_lists(ids, n, E, cnt, off, xrow, where, act, nact, k, kt_moe_wc);
 }
 
-/* the router and the lists in one launch, by one wave (n = M k <= 64 entries, E <= 1024): the top-k of each token
-   leaves entry p's expert in lane p; lane l owns experts 16 l .. 16 l + 15 (counts from the n entries, read with
-   readlane); offsets and the active list by prefix sums over lanes; an entry's place is its expert's offset plus the
-   entries before it with the same expert (ascending flat index, as kt_moe_sort). The same outputs as
-   k_moe_topk + k_moe_sort. */
-__global__ void __launch_bounds__(256) k_moe_route(const float* __restrict__ logits, int M, int E, int k,
+/* the router and the lists in one launch (n = M k <= 64 entries, E <= 1024). The waves take the tokens in turn for the
+   top-k (each token's is one wave's serial chain of k rounds, about 3 us: one wave doing them one after the other took
+   23 us for 7 tokens of 128 experts, 6 picks; one token a wave 5.4 us); the picks meet in LDS, and wave 0 builds the lists
+   while the others quantize x. Lists: lane p holds entry p's expert; the lanes holding the same one found by a ballot a
+   bit of the expert index (an entry's rank among them in lane order, so an expert's entries keep ascending flat index,
+   as kt_moe_sort), their count; lane l owns experts l per .. + per - 1 (per = ceil(E / 64)), offsets and the active list
+   by prefix sums over lanes. The same outputs as k_moe_topk + k_moe_sort. */
+#define KT_RT_WAVES 8
+__global__ void __launch_bounds__(64 * KT_RT_WAVES) k_moe_route(const float* __restrict__ logits, int M, int E, int k,
     const KtRouter rt, int* __restrict__ ids, float* __restrict__ gw, int* __restrict__ cnt, int* __restrict__ off,
     int* __restrict__ xrow, int* __restrict__ where, int* __restrict__ act, int* __restrict__ nact,
     const float* __restrict__ x, int ldx, int H, int8_t* __restrict__ Q, int ldq, float* __restrict__ D, int ldd){
-  __shared__ int o[1024];
-  const int lane = threadIdx.x & 63, n = M * k;
-  if(threadIdx.x >= 64){
-    /* waves 1..3: the tokens' int8 rows, k_quant_q8's numbers (act 0): a 32-lane half per 32-column block */
+  __shared__ int c[1024], o[1024], pick[64];
+  const int lane = threadIdx.x & 63, n = M * k, W = blockDim.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for(int t = w; t < M; t += W){                                   /* wave-uniform */
+    const int mine = kt_topk_wave(logits + (long long)t * E, E, k, rt, ids + t * k, gw + t * k, lane);
+    if(lane < k) pick[t * k + lane] = mine;
+  }
+  for(int e = threadIdx.x; e < E; e += blockDim.x) c[e] = 0;
+  __syncthreads();
+  if(w > 0){
+    /* the other waves: the tokens' int8 rows, k_quant_q8's numbers (act 0): a 32-lane half per 32-column block */
     if(!x) return;
-    /* blocks h, h + 6, ... of every token, KT_RQ at a time: their loads issued together (clamped to a real block),
+    /* blocks h, h + nh, ... of every token, KT_RQ at a time: their loads issued together (clamped to a real block),
        then the reductions and stores, so a half-wave waits for memory once per KT_RQ blocks, not once per block */
-    const int h = (threadIdx.x - 64) >> 5, l = threadIdx.x & 31, nb = H / 32;
+    const int h = (threadIdx.x - 64) >> 5, nh = 2 * (W - 1), l = threadIdx.x & 31, nb = H / 32;
     constexpr int KT_RQ = 8;
     for(int t = 0; t < M; ++t)
-      for(int b0 = h; b0 < nb; b0 += 6 * KT_RQ){
+      for(int b0 = h; b0 < nb; b0 += nh * KT_RQ){
         float v[KT_RQ];
 #pragma unroll
         for(int q = 0; q < KT_RQ; ++q){
-          const int b = b0 + 6 * q;
-          v[q] = x[(long long)t * ldx + (b < nb ? b : h) * 32 + l];
+          const int b = b0 + nh * q;
+          v[q] = x[(long long)t * ldx + (b < nb ? b : b0) * 32 + l];
         }
 #pragma unroll
         for(int q = 0; q < KT_RQ; ++q){
-          const int b = b0 + 6 * q;
+          const int b = b0 + nh * q;
           float a = fabsf(v[q]);
           a = fmaxf(a, kf_xorf<1>(a)); a = fmaxf(a, kf_xorf<2>(a)); a = fmaxf(a, kf_xorf<4>(a));
           a = fmaxf(a, kf_xorf<8>(a)); a = fmaxf(a, kf_xorf<16>(a));
@@ -155,44 +165,47 @@ __global__ void __launch_bounds__(256) k_moe_route(const float* __restrict__ log
       }
     return;
   }
-  int ep = -1;                                                     /* entry lane's expert */
-  for(int t = 0; t < M; ++t){
-    /* entry lanes t k .. t k + k - 1 take the picks from lanes 0 .. k - 1 */
-    const int mine = kt_topk_wave(logits + (long long)t * E, E, k, rt, ids + t * k, gw + t * k, lane);
-    const int got = __builtin_amdgcn_ds_bpermute(((lane - t * k) & 63) << 2, mine);
-    ep = lane >= t * k && lane < t * k + k ? got : ep;
-  }
-  int c[16];
+  const bool valid = lane < n;
+  const int ep = valid ? pick[lane] : 0;
+  unsigned long long eq = __ballot(valid);
 #pragma unroll
-  for(int i = 0; i < 16; ++i) c[i] = 0;
-  for(int q = 0; q < n; ++q){
-    const int d = __builtin_amdgcn_readlane(ep, q) - 16 * lane;
-#pragma unroll
-    for(int i = 0; i < 16; ++i) c[i] += d == i ? 1 : 0;
+  for(int b = 0; b < 10; ++b){
+    const bool bit = (ep >> b) & 1;
+    const unsigned long long bal = __ballot(bit);
+    eq &= bit ? bal : ~bal;
   }
+  const int rank = __popcll(eq & ((1ull << lane) - 1ull));
+  if(valid && rank == 0) c[ep] = __popcll(eq);
+  /* c[] and o[] by this wave only from here: a wave barrier suffices */
+  auto sync = []{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  };
+  sync();
+  const int per = (E + 63) >> 6;
   int tot = 0, na = 0;
-#pragma unroll
-  for(int i = 0; i < 16; ++i){ tot += c[i]; na += c[i] > 0 ? 1 : 0; }
+  for(int i = 0; i < per; ++i){
+    const int e = lane * per + i, ce = e < E ? c[e] : 0;
+    tot += ce;
+    na += ce > 0 ? 1 : 0;
+  }
   int tall, all;
   int base = kt_wave_excl_scan(tot, lane, &tall), abase = kt_wave_excl_scan(na, lane, &all);
-#pragma unroll
-  for(int i = 0; i < 16; ++i){
-    const int e = 16 * lane + i;
+  for(int i = 0; i < per; ++i){
+    const int e = lane * per + i;
     if(e < E){
-      cnt[e] = c[i];
+      const int ce = c[e];
+      cnt[e] = ce;
       off[e] = base;
       o[e] = base;
-      if(c[i] > 0) act[abase++] = e;
+      if(ce > 0) act[abase++] = e;
+      base += ce;
     }
-    base += c[i];
   }
   if(lane == 0) *nact = all;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");        /* o[] by this wave only: a wave barrier suffices */
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  if(lane < n){
-    int rank = 0;
-    for(int q = 0; q < n; ++q) rank += (q < lane && __builtin_amdgcn_readlane(ep, q) == ep) ? 1 : 0;
+  sync();
+  if(valid){
     const int pos = o[ep] + rank;
     xrow[pos] = lane / k;
     where[lane] = pos;
