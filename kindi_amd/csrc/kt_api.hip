@@ -37,17 +37,17 @@ template <bool HP> __global__ void k_quant_tern(const float*, int, int, int, int
 template <int NR> __global__ void k_quant_row(const float*, int, int, int8_t*, int, float*, int*);
 extern "C" __global__ void k_quant_q8(const float*, int, int, int, int8_t*, int, float*, int);
 extern "C" __global__ void k_tern_sum(const float*, float*, int, int, int);
-template <bool DBG, bool RS>
-__global__ void k_tern_gemm(const uint32_t*, const uint16_t*, int, int, const int8_t*, int, const float*, int, float*,
-                            uint16_t*, int, int32_t*);
+template <bool RS, bool DBG>
+__global__ void k_tern_gemm_ks(const uint32_t*, const uint16_t*, int, int, const int8_t*, int, const float*, int, float*,
+                               uint16_t*, int, int32_t*, int, int);
+template <int T, bool RS, bool DBG>
+__global__ void k_tern_gemm_w(const uint32_t*, const uint16_t*, int, int, const int8_t*, int, const float*, int, float*,
+                              uint16_t*, int, int32_t*, int, int);
 extern "C" __global__ void k_tern_expand(const uint4*, int, long long, int, int8_t*);
 template <bool DBG>
 __global__ void k_tern_gemm8(const int8_t*, const uint16_t*, int, int, const int8_t*, int, const float*, int, float*,
                              uint16_t*, int, int32_t*, int, int);
 size_t kt_gemm8_lds();
-template <int WT, int WR, int PD, bool DBG>
-__global__ void k_tern_gemm_rs1(const uint32_t*, const uint16_t*, int, int, const int8_t*, int, const float*, int,
-                                float*, uint16_t*, int, int32_t*);
 __global__ void k_moe_topk(const float*, int, int, const KtRouter, int*, float*);
 extern "C" __global__ void k_moe_sort(const int*, int, int, int*, int*, int*, int*, int*, int*, int);
 extern "C" __global__ void k_moe_combine(const float*, const float*, const int*, const float*, int, int, float*, int);
@@ -80,7 +80,6 @@ size_t kt_moe1_down_lds(int k, int KS);
 #define KT_PAIR_WAVES 6144             /* one-token grids of more waves take two row groups a block (k_gemv_pair) */
 #endif
 #define KT_RT_BLOCK 512                /* k_moe_route's threads (kt_moe.hip KT_RT_WAVES waves) */
-#define KT_RS_BLOCKS 1024              /* per-row prefill on small blocks while the 128 x 128 grid has fewer blocks */
 
 static inline hipStream_t kt_stream(void* s){ return (hipStream_t)s; }
 static inline bool kt_al(const void* p, size_t a){ return ((uintptr_t)p % a) == 0; }
@@ -556,43 +555,6 @@ int kt_tern_sum(const float* P, float* y, int R, int M, int sp, void* stream){
 }
 
 
-/* ------------------------------------------------------------------ prefill product */
-/* per_row = 0: the reference's per-group expression on 128 x 128 blocks. per_row = 1: the per-row order, on small
-   blocks (128 tokens x 64 rows) while a grid of 128 x 128 blocks would have fewer than KT_RS_BLOCKS blocks (4 a CU),
-   else on 128 x 128 blocks; both run the same per-element chain, so the bits do not depend on the choice (measured
-   on MI355X, config 2: gate/up [12288 x 4096] at 512 tokens 60.0 -> 56.5 us on the small blocks, at 2048 tokens
-   190.8 against 202.6 us on the large ones) */
-int kt_tern_gemm(const void* W, int R, int C, const int8_t* XQ, int ldq, const float* XS, const int32_t* XA,
-                 int per_row, int M, float* Y, uint16_t* Y16, int ldy, int32_t* dbg, void* stream){
-  (void)XA;                                                  /* signed trits on the matrix cores: no digit offset */
-  if(M == 0) return 0;
-  if(!W || !XQ || !XS || (!Y && !Y16) || R <= 0 || M < 0 || C <= 0 || C % 128 || ldq < C || ldq % 16 || ldy < R
-     || !kt_al(W, 16) || !kt_al(XQ, 16) || (per_row != 0 && per_row != 1)) return KT_INVALID;
-  const int NG = C / 128;
-  const uint32_t* codes = (const uint32_t*)W;
-  const uint16_t* scales = (const uint16_t*)((const uint8_t*)W + kt_code_bytes(R, NG));
-  /* both kernels read through buffer resources with 32-bit offsets */
-  if((long long)M * ldq >= (1ll << 31) || (long long)M * NG * 4 >= (1ll << 31) || kt_code_bytes(R, NG) >= (1ull << 31))
-    return KT_INVALID;
-  hipStream_t s = kt_stream(stream);
-  if(per_row && (long long)((R + 127) / 128) * ((M + 127) / 128) < KT_RS_BLOCKS){
-    /* one 32 x 32 tile a wave, 8 waves: 128 tokens x 64 rows */
-    const dim3 grid((R + 63) / 64, (M + 127) / 128);
-    if(dbg) KT_LAUNCH((k_tern_gemm_rs1<4, 2, 3, true>), grid, dim3(512), 0, s, codes, scales, R, NG, XQ, ldq,
-                               XS, M, Y, Y16, ldy, dbg);
-    else KT_LAUNCH((k_tern_gemm_rs1<4, 2, 3, false>), grid, dim3(512), 0, s, codes, scales, R, NG, XQ, ldq,
-                            XS, M, Y, Y16, ldy, dbg);
-    return 0;
-  }
-  const dim3 grid((R + 127) / 128, (M + 127) / 128);
-#define KT_TG(DBG, RS) KT_LAUNCH((k_tern_gemm<DBG, RS>), grid, dim3(256), 0, s, codes, scales, R, NG, XQ, ldq, \
-                                          XS, M, Y, Y16, ldy, dbg)
-  if(per_row){ if(dbg) KT_TG(true, true); else KT_TG(false, true); }
-  else { if(dbg) KT_TG(true, false); else KT_TG(false, false); }
-#undef KT_TG
-  return 0;
-}
-
 /* the current device's CU count, queried once per device */
 static int kt_cu_count(int* cus){
   static int cache[64];
@@ -607,6 +569,50 @@ static int kt_cu_count(int* cus){
     cache[dev] = n;
   }
   *cus = cache[dev];
+  return 0;
+}
+
+/* ------------------------------------------------------------------ prefill product */
+/* Which kernel, by how many 32 x 32 output tiles the launch has (every one runs the same per-element chain, so the bits
+   do not depend on the choice; MI355X, 256 CUs, group scales):
+   - up to 2 a CU: k_tern_gemm_ks, a tile a block with its groups dealt over 4 waves (two such blocks share a CU):
+     [5120 x 5120] at 61 / 96 tokens (320 / 480 tiles) 13.0 / 13.7 against 18.6 / 19.0 us for k_tern_gemm_w<1>, [4096 x
+     12288] at 128 (512) 28 against 40; past it [5120 x 5120] at 128 (640) 19.9 against 19.1, [17408 x 5120] at 61
+     (1088) 30 against 24;
+   - k_tern_gemm_w<1>, one tile a wave, up to 12 tiles (3 blocks) a CU: [17408 x 5120] at 128 tokens (2176) 32.0
+     against 34.8 us for two tiles a wave, [12288 x 4096] at 256 (3072) 27.1 against 29.6;
+   - above, k_tern_gemm_w<2>: [17408 x 5120] at 256 tokens (4352) 47.4 against 50.7, [4096 x 12288] at 1000 (4096) 81
+     against 93. */
+int kt_tern_gemm(const void* W, int R, int C, const int8_t* XQ, int ldq, const float* XS, const int32_t* XA,
+                 int per_row, int M, float* Y, uint16_t* Y16, int ldy, int32_t* dbg, void* stream){
+  (void)XA;                                                  /* signed trits on the matrix cores: no digit offset */
+  if(M == 0) return 0;
+  if(!W || !XQ || !XS || (!Y && !Y16) || R <= 0 || M < 0 || C <= 0 || C % 128 || ldq < C || ldq % 16 || ldy < R
+     || !kt_al(W, 16) || !kt_al(XQ, 16) || (per_row != 0 && per_row != 1)) return KT_INVALID;
+  const int NG = C / 128;
+  const uint32_t* codes = (const uint32_t*)W;
+  const uint16_t* scales = (const uint16_t*)((const uint8_t*)W + kt_code_bytes(R, NG));
+  /* the kernels read through buffer resources with 32-bit offsets */
+  if((long long)M * ldq >= (1ll << 31) || (long long)M * NG * 4 >= (1ll << 31) || kt_code_bytes(R, NG) >= (1ull << 31))
+    return KT_INVALID;
+  hipStream_t s = kt_stream(stream);
+  int cus = 0;
+  const int ec = kt_cu_count(&cus);
+  if(ec) return ec;
+  const long long rt = (R + 31) / 32, tt = (M + 31) / 32, tiles = rt * tt;
+  const int gx = (R + 127) / 128;
+#define KT_PF(K, GX, GY) KT_LAUNCH((K), dim3((unsigned)((GX) * (GY))), dim3(256), 0, s, codes, scales, R, NG, XQ, ldq, XS, \
+                                   M, Y, Y16, ldy, dbg, (int)(GX), (int)(GY))
+#define KT_PFS(K, GX, GY, ...) do { \
+    if(per_row){ if(dbg) KT_PF((K<__VA_ARGS__ true, true>), GX, GY); else KT_PF((K<__VA_ARGS__ true, false>), GX, GY); } \
+    else { if(dbg) KT_PF((K<__VA_ARGS__ false, true>), GX, GY); else KT_PF((K<__VA_ARGS__ false, false>), GX, GY); } } while(0)
+#define KT_COMMA ,
+  if(tiles <= 2ll * cus) KT_PFS(k_tern_gemm_ks, rt, tt, );
+  else if(gx * tt <= 3ll * cus) KT_PFS(k_tern_gemm_w, gx, tt, 1 KT_COMMA);
+  else KT_PFS(k_tern_gemm_w, gx, (M + 63) / 64, 2 KT_COMMA);
+#undef KT_COMMA
+#undef KT_PFS
+#undef KT_PF
   return 0;
 }
 

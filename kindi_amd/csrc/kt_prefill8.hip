@@ -25,10 +25,10 @@
    131 against 199 us, down [4096 x 12288] 128 against 172 us (with two-byte stores straight from the accumulators:
    175 and 142 us). Below one block a CU (M = 512) the packed-trit kernels are faster and kt_tern_gemm8 runs them. */
 #include "kt_common.h"
+#include "kt_dma.h"
 
 typedef int kt8_v4i __attribute__((ext_vector_type(4)));
 typedef int kt8_v16i __attribute__((ext_vector_type(16)));
-#define KT_L3 __attribute__((address_space(3)))
 
 #define P8_BT 128                     /* tokens a block */
 #define P8_BR 256                     /* weight rows a block */
@@ -65,27 +65,6 @@ extern "C" __global__ void __launch_bounds__(256) k_tern_expand(const uint4* __r
 }
 
 /* ------------------------------------------------------------------ the product */
-/* a buffer resource as the 4 dwords the asm takes: base, stride 0, num_records bytes, gfx950 default flags */
-__device__ __forceinline__ kt8_v4i p8_rsrc(const void* p, uint32_t bytes){
-  const unsigned long long a = (unsigned long long)p;
-  kt8_v4i r;
-  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-  r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32) & 0xFFFF);
-  r.z = (int)bytes;
-  r.w = 0x00020000;
-  return r;
-}
-/* DMA: lane i's 16 bytes at byte voff of the buffer land at LDS byte address lds + 16 i (lds wave-uniform); an offset
-   past the buffer lands zeros */
-__device__ __forceinline__ void p8_dma(kt8_v4i rs, uint32_t voff, uint32_t lds){
-  const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               :: "s"(l), "v"(voff), "s"(rs) : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t p8_lds(const void* p){
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(const KT_L3 void*)p);
-}
-
 template <bool DBG>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 k_tern_gemm8(const int8_t* __restrict__ W8, const uint16_t* __restrict__ scales, int R, int C, const int8_t* __restrict__ XQ,
@@ -95,10 +74,10 @@ k_tern_gemm8(const int8_t* __restrict__ W8, const uint16_t* __restrict__ scales,
   const int NG = C >> 7, R8 = kt_r8(R), ntiles = gx * gy;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), wt = w & 1, wr = w >> 1;
   const uint32_t OOB = 0x80000000u;
-  const kt8_v4i rx = p8_rsrc(XQ, (uint32_t)M * (uint32_t)ldq);
-  const kt8_v4i rw = p8_rsrc(W8, (uint32_t)R8 * 8u * (uint32_t)C);
-  const kt8_v4i rh = p8_rsrc(scales, (uint32_t)R8 * (uint32_t)NG * 16u);
-  const uint32_t lbase = p8_lds(p8_lds_buf);
+  const kt8_v4i rx = kt_dma_rsrc(XQ, (uint32_t)M * (uint32_t)ldq);
+  const kt8_v4i rw = kt_dma_rsrc(W8, (uint32_t)R8 * 8u * (uint32_t)C);
+  const kt8_v4i rh = kt_dma_rsrc(scales, (uint32_t)R8 * (uint32_t)NG * 16u);
+  const uint32_t lbase = kt_dma_lds(p8_lds_buf);
   /* DMA instruction i of a wave takes rows 8 i + lane / 8 (+ 16 w activations, + 32 w trits) of the tile, chunk
      (lane % 8) ^ ((row >> 1) & 7) = (lane % 8) ^ ((lane / 8) >> 1) ^ 4 (i & 1): one source offset for the rows of even
      i and one for odd i. Rows past M or past the padded rows read past their buffer (zeros: row * stride is at least
@@ -136,10 +115,10 @@ k_tern_gemm8(const int8_t* __restrict__ W8, const uint16_t* __restrict__ scales,
   auto issue = [&](int g){
     const uint32_t st = lbase + (uint32_t)((g % P8_NS) * P8_STAGE);
 #pragma unroll
-    for(int i = 0; i < 2; ++i) p8_dma(rx, xo[i & 1] + (uint32_t)(8 * i * ldq + g * 128), st + (16 * w + 8 * i) * 128);
+    for(int i = 0; i < 2; ++i) kt_dma16(rx, xo[i & 1] + (uint32_t)(8 * i * ldq + g * 128), 0, st + (16 * w + 8 * i) * 128);
 #pragma unroll
-    for(int i = 0; i < 4; ++i) p8_dma(rw, wo[i & 1] + (uint32_t)(8 * i * C + g * 128), st + P8_A + (32 * w + 8 * i) * 128);
-    if(lane < 4) p8_dma(rh, so + (uint32_t)g * 16u, st + P8_A + P8_W + 64 * w);
+    for(int i = 0; i < 4; ++i) kt_dma16(rw, wo[i & 1] + (uint32_t)(8 * i * C + g * 128), 0, st + P8_A + (32 * w + 8 * i) * 128);
+    if(lane < 4) kt_dma16(rh, so + (uint32_t)g * 16u, 0, st + P8_A + P8_W + 64 * w);
   };
   /* the top of group g: this wave's DMAs of group g have landed when at most group g + 1's are in flight (loads retire
      in order, so the pending ones are the last issued; stores issued before them do not matter); after the barrier

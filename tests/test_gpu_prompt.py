@@ -1,0 +1,73 @@
+"""The prefill product's kernels at the edges of their dispatch (kt_tern_gemm): a tile a block with its groups dealt over
+4 waves (up to 2 tiles of 32 x 32 a CU), one tile a wave (up to 12), two tiles a wave. Every one applies the reference
+expression group after group, so the int32 group values and the fp32 outputs are the oracle's, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as orc
+from kt_cases import say, tern_case, dev, host, rng
+
+pytestmark = pytest.mark.gpu
+
+
+def _tiles(R, M):
+    return -(-R // 32) * -(-M // 32)
+
+
+def _route(R, M):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if _tiles(R, M) <= 2 * cus:
+        return "split"
+    return "one" if -(-R // 128) * -(-M // 32) <= 3 * cus else "two"
+
+
+# group counts around the 4 groups of a round, the 3 stages and the 8 units of a kt2 step; ragged rows and tokens
+@pytest.mark.parametrize("R,C,M,route", [
+    (8, 128, 1, "split"), (40, 256, 17, "split"), (100, 384, 33, "split"), (31, 512, 64, "split"), (65, 640, 31, "split"),
+    (257, 1152, 45, "split"), (96, 1664, 96, "split"), (5120, 1408, 61, "split"),
+    (8200, 128, 70, "one"), (8200, 256, 95, "one"), (8193, 384, 65, "one"), (8260, 512, 100, "one"), (8300, 1152, 97, "one"),
+    (8200, 128, 400, "two"), (8197, 256, 385, "two"), (8200, 384, 449, "two"), (8300, 1280, 390, "two")])
+@pytest.mark.parametrize("per_row", [False, True])
+def test_gemm_routes(R, C, M, route, per_row):
+    from kindi_amd import linear
+    say("gemm route", R, C, M, route, per_row)
+    assert _route(R, M) == route
+    dig, bc, dpm = tern_case(R, C, R + C + M)
+    L = linear.Linear({"w": linear.TernaryMatrix(bc, dpm, R, C)})
+    X = rng(M + 5).normal(0, 1, (M, C)).astype(np.float32)
+    act = linear.quantize(dev(X), per_row=per_row)
+    Q, XS, XA = orc.quant_q8(X, per_row=per_row)
+    acc = orc.tern_acc(bc, R, C, Q)
+    want = (orc.tern_out_rs if per_row else orc.tern_out)(acc, XS, dpm, R, C)
+    dbg = torch.empty((M, R, C // 128), dtype=torch.int32, device="cuda")
+    Y = torch.empty((M, R), dtype=torch.float32, device="cuda")
+    Y16 = torch.empty((M, R), dtype=torch.float16, device="cuda")
+    L.gemm("w", act, Y=Y, Y16=Y16, dbg=dbg)
+    assert np.array_equal(host(dbg), acc), "int32 group values"
+    assert np.array_equal(host(Y), want), "debug instantiation"
+    assert np.array_equal(host(Y16), want.astype(np.float16))
+    assert np.array_equal(host(L.gemm("w", act)), want)
+    wide = torch.full((M, R + 3), -7.0, device="cuda")                    # rows of a wider buffer: the pad untouched
+    L.gemm("w", act, Y=wide[:, :R])
+    assert np.array_equal(host(wide[:, :R]), want) and bool((wide[:, R:] == -7.0).all())
+
+
+@pytest.mark.parametrize("R,M,route", [(256, 64, "split"), (8200, 70, "one"), (8200, 400, "two")])
+def test_gemm_scale_extremes(R, M, route):
+    """token scales whose product with a row scale is subnormal, overflows, or is not a number: the element scale is
+    XS d rounded once on every route (the two-tile route makes it on the matrix cores)"""
+    from kindi_amd import linear
+    say("gemm scales", R, M, route)
+    assert _route(R, M) == route
+    C = 384
+    dig, bc, dpm = tern_case(R, C, 77)
+    L = linear.Linear({"w": linear.TernaryMatrix(bc, dpm, R, C)})
+    act = linear.quantize(dev(rng(3).normal(0, 1, (M, C)).astype(np.float32)))
+    sc = np.array([1e-38, 3e-40, 1.4e-45, 0.0, 2e38, np.inf, np.nan, 1.0, -0.5, 1.1754944e-38], np.float32)
+    act.XS.copy_(dev(np.tile(sc, (M * (C // 128) + 9) // 10)[:M * (C // 128)].reshape(M, C // 128)))
+    with np.errstate(all="ignore"):
+        want = orc.tern_out(orc.tern_acc(bc, R, C, host(act.XQ)), host(act.XS), dpm, R, C)
+    got = host(L.gemm("w", act))
+    same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+    assert same.all(), (int((~same).sum()), got[~same][:4], want[~same][:4])
