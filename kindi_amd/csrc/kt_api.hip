@@ -30,6 +30,8 @@ template <bool DBG, int KQ, bool MS>
 __global__ void k_gemv_m16(const KtGemvArgs, const int8_t*, const float*, const int*, int32_t*, int);
 template <bool GRP, bool DBG, bool MS>
 __global__ void k_q8_mma(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
+template <bool GRP, bool DBG>
+__global__ void k_q8_gemm(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
 template <int SRC> __global__ void k_tern_pack(const uint8_t*, const uint16_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_q8_pack(const uint8_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_tern_pack_ptq1(const uint8_t*, int, int, int, int, uint32_t*, uint16_t*);
@@ -94,6 +96,9 @@ static int kt_kslices(int NU){
   return ks < KT_KSMAX ? ks : KT_KSMAX;
 }
 
+/* k_q8_gemm holds slices of one or two steps (rows of up to 8192 columns: beyond, 16 slices are longer) */
+static bool kt_q8_gemm_takes(int NU){ return kt_steps(NU) <= KT_SL * kt_kslices(NU); }
+
 /* up to 32 ternary tokens: the matrix-core product (the same numbers and tree, so the same bits), tiles of 32 rows
    of one matrix, passes of 16 tokens, on every launch from 3 tokens (measured on MI355X with k_gemv_m16 and its
    k-lanes split over 4 waves on small grids, per launch over 16 27B-class layers and per 2B-class layer: 27B layer
@@ -104,7 +109,6 @@ static int kt_kslices(int NU){
 #ifndef KT_MMA_MIN
 #define KT_MMA_MIN 3
 #endif
-#define KT_Q8_MMA_MIN 12               /* q8_0 dense: the matrix-core product from 12 tokens */
 #define KT_MMA_MAX 32
 #define KT_Q8_MMA_KS 8                 /* q8_0 matrix-core product: K slices a block (kt_mma.hip KM_Q8_KS) */
 #ifndef KT_MMA_W2
@@ -423,6 +427,23 @@ hipError_t kt_rec_push(const void* fn, dim3 g, dim3 b, size_t lds, int n, const 
   return hipSuccess;
 }
 
+/* the current device's CU count, queried once per device */
+static int kt_cu_count(int* cus){
+  static int cache[64];
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if(e != hipSuccess) return (int)e;
+  if(dev < 0 || dev >= 64) return KT_INVALID;
+  if(!cache[dev]){
+    int n = 0;
+    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    if(e != hipSuccess) return (int)e;
+    cache[dev] = n;
+  }
+  *cus = cache[dev];
+  return 0;
+}
+
 extern "C" {
 
 int kt_version(void){ return KT_VERSION; }
@@ -554,23 +575,6 @@ int kt_tern_sum(const float* P, float* y, int R, int M, int sp, void* stream){
   return 0;
 }
 
-
-/* the current device's CU count, queried once per device */
-static int kt_cu_count(int* cus){
-  static int cache[64];
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if(e != hipSuccess) return (int)e;
-  if(dev < 0 || dev >= 64) return KT_INVALID;
-  if(!cache[dev]){
-    int n = 0;
-    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    if(e != hipSuccess) return (int)e;
-    cache[dev] = n;
-  }
-  *cus = cache[dev];
-  return 0;
-}
 
 /* ------------------------------------------------------------------ prefill product */
 /* Which kernel, by how many 32 x 32 output tiles the launch has (every one runs the same per-element chain, so the bits
@@ -712,11 +716,36 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
   a.ldq = ldq; a.ldxs = ldd;
   a.M = M;
   const int ks = kt_kslices(NB);
-  if(M >= KT_Q8_MMA_MIN && ks <= KT_Q8_MMA_KS && (long long)M * ldq < (1ll << 31)){
-    /* the matrix-core product (the same numbers and tree): tiles of 32 rows, all tokens a block */
-    const dim3 grid((kt_r8(R) + 3) / 4), block(64 * ks);
+  const KtGroupedArgs ga = {};
+  /* Which kernel (all the same numbers and tree; MI355X, weights from HBM):
+     - the matrix cores with a K slice a wave (k_q8_mma, up to 8 slices) from 9 tokens, from 5 on 2^22 weights, from 3 on
+       2^25: [2688 x 1856] at 4 / 5 tokens 6.4 against 7.4 / 8.3 -> 7.3 us, [8192 x 4096] at 3 tokens 14.2 -> 11.5,
+       [1024 x 1024] at 5 / 10 tokens 6.1 against 6.8 / 8.1 -> 6.9;
+     - k_q8_gemm above 10 (tile of 32 rows, pass of 16 tokens) pairs a CU: [4096 x 2688] at 256 / 600 tokens (2048 / 4864
+       pairs) 33 against 41 / 70 -> 52 us, [8192 x 4096] at 128 / 256 (2048 / 4096) 47 against 54 / 87 -> 56; and from 64
+       tokens where the rows have more than 8 slices: [4096 x 8192] at 50 / 100 tokens 117 / 217 against 98 / 99 us,
+       [1024 x 5120] 42 / 76 against 63 / 63;
+     - the v_dot4 kernel else. */
+  int cus = 0;
+  const int ec = kt_cu_count(&cus);
+  if(ec) return ec;
+  const int tiles = (kt_r8(R) + 3) / 4, np = M / 16 + (M % 16 ? 1 : 0);
+  const long long nw = (long long)R * C;
+  if((ks <= KT_Q8_MMA_KS ? (long long)tiles * np > 10ll * cus : M >= 64) && kt_q8_gemm_takes(NB)
+     && (long long)M * ldq < (1ll << 31)
+     && (long long)M * ldd * 4 < (1ll << 31) && (long long)kt_r8(R) * NB * 272 < (1ll << 31) && (M + 63) / 64 <= 65535){
+    const dim3 grid((R + 127) / 128, (M + 63) / 64);
+    if(dbg) KT_LAUNCH((k_q8_gemm<false, true>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks);
+    else KT_LAUNCH((k_q8_gemm<false, false>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks);
+    return 0;
+  }
+  if((M >= 9 || (M >= 5 && nw >= 1ll << 22) || (M >= 3 && nw >= 1ll << 25)) && ks <= KT_Q8_MMA_KS
+     && (long long)M * ldq < (1ll << 31)){
+    /* tiles of 32 rows, the passes of 16 tokens dealt over as many blocks as give each CU one (of ks waves, 256 registers a
+       lane): [4096 x 2688] at 50 tokens 18.7 -> 12.6 us, [1024 x 1024] at 128 25.4 -> 7.5; two a CU was no faster */
+    const int want = (cus + tiles - 1) / tiles, gy = want < np ? want : np;
+    const dim3 grid(tiles, gy), block(64 * ks);
     const size_t lds = (size_t)ks * 16 * 32 * 4 + (size_t)ks * 256 * 4;          /* slice sums, D */
-    const KtGroupedArgs ga = {};
     if(dbg) KT_LAUNCH((k_q8_mma<false, true, false>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
     else KT_LAUNCH((k_q8_mma<false, false, false>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
     return 0;
@@ -791,6 +820,19 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
   const int ks = kt_kslices(a.NU);
   const int ny = E < nentries ? E : nentries;
   hipStream_t s = kt_stream(stream);
+  /* 10 or more entries an expert on average: k_q8_gemm, whose two tiles of 32 entries a wave share the weights (MI355X, 128
+     experts, 6 picks, up [1856 x 2688] / down [2688 x 1856]: at 96 entries 1003 / 976 -> 398 / 391 us, 24: 310 / 304 -> 174
+     / 179, 12: 181 / 172 -> 158 / 168, but 9: 152 / 151 against 153 / 164); from 4 where the rows have more slices than
+     k_q8_mma takes */
+  const bool off32 = (long long)a.nrows * ldq < (1ll << 31) && (long long)a.nrows * ldd * 4 < (1ll << 31)
+                     && (long long)kt_r8(R) * a.NU * 272 < (1ll << 31);
+  if(nentries >= (ks <= KT_Q8_MMA_KS ? 10ll : 4ll) * ny && off32 && kt_q8_gemm_takes(a.NU)){
+    const dim3 grid((R + 127) / 128, ny);
+    const KtGemvArgs da = {};
+    if(dbg) KT_LAUNCH((k_q8_gemm<true, true>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks);
+    else KT_LAUNCH((k_q8_gemm<true, false>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks);
+    return 0;
+  }
   /* the matrix-core kernel reads the input rows through a buffer resource with 32-bit offsets */
   if(nentries >= 4 * ny && ks <= KT_Q8_MMA_KS && (long long)a.nrows * ldq < (1ll << 31)){
     /* 4 or more entries an active expert on average: the matrix-core product per (32-row tile, active expert), the

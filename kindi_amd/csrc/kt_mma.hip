@@ -633,14 +633,16 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
     /* one slice a wave, its weights loaded once for every pass: the input rows of pass 0, then the weights
        (independent of them), then the pass's D and activations, so the weight stream overlaps the list
        indirection; each pass issues the next pass's loads before its slice sums */
-    ld_rows(0);
+    const int tb = GRP ? 0 : blockIdx.y * NT, ts = GRP ? NT : gridDim.y * NT;      /* dense: passes blockIdx.y, + gridDim.y .. */
+    if(tb >= cntM) return;                                       /* uniform */
+    ld_rows(tb);
     __builtin_amdgcn_sched_barrier(0);
     ld_w();
     __builtin_amdgcn_sched_barrier(0);
-    ld_pass(0);
-    for(int t0 = 0; t0 < cntM; t0 += NT){                        /* uniform: the block's list in passes */
+    ld_pass(tb);
+    for(int t0 = tb; t0 < cntM; t0 += ts){                        /* uniform: the block's list in passes */
       compute(t0);
-      if(t0 + NT < cntM){ ld_rows(t0 + NT); ld_pass(t0 + NT); }  /* uniform: the next pass's loads in flight */
+      if(t0 + ts < cntM){ ld_rows(t0 + ts); ld_pass(t0 + ts); }  /* uniform: the next pass's loads in flight */
       finish(t0);
     }
   } else {
