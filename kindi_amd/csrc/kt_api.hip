@@ -31,7 +31,7 @@ __global__ void k_gemv_m16(const KtGemvArgs, const int8_t*, const float*, const 
 template <bool GRP, bool DBG, bool MS>
 __global__ void k_q8_mma(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
 template <bool GRP, bool DBG>
-__global__ void k_q8_gemm(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
+__global__ void k_q8_gemm(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int, int);
 template <int SRC> __global__ void k_tern_pack(const uint8_t*, const uint16_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_q8_pack(const uint8_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_tern_pack_ptq1(const uint8_t*, int, int, int, int, uint32_t*, uint16_t*);
@@ -735,8 +735,8 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
      && (long long)M * ldq < (1ll << 31)
      && (long long)M * ldd * 4 < (1ll << 31) && (long long)kt_r8(R) * NB * 272 < (1ll << 31) && (M + 63) / 64 <= 65535){
     const dim3 grid((R + 127) / 128, (M + 63) / 64);
-    if(dbg) KT_LAUNCH((k_q8_gemm<false, true>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks);
-    else KT_LAUNCH((k_q8_gemm<false, false>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks);
+    if(dbg) KT_LAUNCH((k_q8_gemm<false, true>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks, 1);
+    else KT_LAUNCH((k_q8_gemm<false, false>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks, 1);
     return 0;
   }
   if((M >= 9 || (M >= 5 && nw >= 1ll << 22) || (M >= 3 && nw >= 1ll << 25)) && ks <= KT_Q8_MMA_KS
@@ -827,10 +827,15 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
   const bool off32 = (long long)a.nrows * ldq < (1ll << 31) && (long long)a.nrows * ldd * 4 < (1ll << 31)
                      && (long long)kt_r8(R) * a.NU * 272 < (1ll << 31);
   if(nentries >= (ks <= KT_Q8_MMA_KS ? 10ll : 4ll) * ny && off32 && kt_q8_gemm_takes(a.NU)){
-    const dim3 grid((R + 127) / 128, ny);
+    /* P blocks share a row tile's passes of 64, so that a long list (a popular expert) does not hold one block's CU to the
+       end: router scores with a bias of 0.1 N(0, 1), 96 entries an expert, P 1 / 3 / 7: up 678 / 471 / 427 us, 48: 360 / 287
+       / 260; without the bias 396 / 385 / 392. Odd: the blocks past a list's end leave at once, and an even P left the same
+       half of the shader engines with them (P 2 and 4 at 96 entries: 422 and 745 us) */
+    const int P = nentries / ny < 64 ? 3 : 7;
+    const dim3 grid((unsigned)(((long long)((R + 127) / 128) * ny + 7) / 8 * 8 * P));
     const KtGemvArgs da = {};
-    if(dbg) KT_LAUNCH((k_q8_gemm<true, true>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks);
-    else KT_LAUNCH((k_q8_gemm<true, false>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks);
+    if(dbg) KT_LAUNCH((k_q8_gemm<true, true>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P);
+    else KT_LAUNCH((k_q8_gemm<true, false>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P);
     return 0;
   }
   /* the matrix-core kernel reads the input rows through a buffer resource with 32-bit offsets */

@@ -53,26 +53,34 @@ __device__ __forceinline__ void qg_ldw(const __amdgpu_buffer_rsrc_t rw, int c, i
 
 template <bool GRP, bool DBG>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 1 : 2))) k_q8_gemm(const KtGemvArgs a,
-    const KtGroupedArgs ga, const int8_t* __restrict__ xq, const float* __restrict__ xd, int32_t* __restrict__ dbg, int KS){
+    const KtGroupedArgs ga, const int8_t* __restrict__ xq, const float* __restrict__ xd, int32_t* __restrict__ dbg, int KS, int P){
   __shared__ __attribute__((aligned(16))) KtQg L;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, n = lane & 31;
   const uint8_t* wbuf;
   float* yout;
-  int R, NU, ldy, ldq, ldd, nrows, t_lo, t_hi, p0 = 0;
+  int R, NU, ldy, ldq, ldd, nrows, t_lo, t_hi, t_st, p0 = 0, bx;
   const int* xrow = nullptr;
   if(GRP){
-    const int nact = *ga.nact, e = __builtin_amdgcn_readfirstlane(ga.act[blockIdx.y]);
-    if((int)blockIdx.y >= nact) return;
+    /* blocks of one row tile, P of them (passes z, z + P, ..), 8 ids apart: on one XCD at one time, so that its L2 serves
+       the weights to all but the first */
+    const int gx = (ga.R + 127) >> 7, z = (int)(blockIdx.x >> 3) % P;
+    const int tile = ((int)(blockIdx.x >> 3) / P) * 8 + (int)(blockIdx.x & 7), ie = tile / gx;
+    bx = tile - ie * gx;
+    const int nact = *ga.nact;
+    if(ie >= nact) return;
+    const int e = __builtin_amdgcn_readfirstlane(ga.act[ie]);
     wbuf = ga.wexp[e];
     R = ga.R; NU = ga.NU; ldy = ga.ldy; ldq = ga.ldq; ldd = ga.ldd; nrows = ga.nrows; xrow = ga.xrow; yout = ga.y;
-    p0 = __builtin_amdgcn_readfirstlane(ga.off[e]); t_lo = 0; t_hi = __builtin_amdgcn_readfirstlane(ga.cnt[e]);
+    p0 = __builtin_amdgcn_readfirstlane(ga.off[e]); t_hi = __builtin_amdgcn_readfirstlane(ga.cnt[e]);
+    t_lo = z * QG_T; t_st = P * QG_T;
+    if(t_lo >= t_hi) return;
   } else {
     wbuf = (const uint8_t*)a.mat[0].codes;
     R = a.mat[0].R; NU = a.NU; ldy = a.mat[0].ldy; ldq = a.ldq; ldd = a.ldxs; nrows = a.M; yout = a.mat[0].y;
-    t_lo = blockIdx.y * QG_T; t_hi = min(a.M, t_lo + QG_T);
+    bx = blockIdx.x; t_lo = blockIdx.y * QG_T; t_hi = min(a.M, t_lo + QG_T); t_st = QG_T;
   }
-  const int R8 = kt_r8(R), S = kt_steps(NU), row = blockIdx.x * 128 + 32 * w + n, rg = row >> 3;
+  const int R8 = kt_r8(R), S = kt_steps(NU), row = bx * 128 + 32 * w + n, rg = row >> 3;
   const uint32_t OOB = 0x80000000u;
   const kt_v4i rx = kt_dma_rsrc(xq, (uint32_t)nrows * (uint32_t)ldq);
   const kt_v4i rs = kt_dma_rsrc(xd, (uint32_t)nrows * (uint32_t)ldd * 4u);
@@ -176,7 +184,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
       kt_dma4(rs, rd != OOB && u < NU && uc < 8 * ns ? rd + (uint32_t)u * 4u : OOB, 0, lx + st * 2048 + i * 256);
     }
   };
-  for(int t0 = t_lo; t0 < t_hi; t0 += QG_T){
+  for(int t0 = t_lo; t0 < t_hi; t0 += t_st){
     const int nt = min(QG_T, t_hi - t0), T = nt > 32 ? 2 : 1;
     if(tid < QG_T){
       const int p = p0 + t0 + tid;
@@ -210,5 +218,5 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
 }
 
 #define KT_QG(GRP, DBG) template __global__ void k_q8_gemm<GRP, DBG>(const KtGemvArgs, const KtGroupedArgs, const int8_t*, \
-    const float*, int32_t*, int);
+    const float*, int32_t*, int, int);
 KT_QG(false, false) KT_QG(false, true) KT_QG(true, false) KT_QG(true, true)
