@@ -25,8 +25,14 @@ def ptr(t):
     return VP(t.data_ptr()) if t is not None else None
 
 
+def _raw_stream():
+    """the current stream's handle. torch.cuda.current_stream() builds a Stream object (2.8 us a call on the measured
+    host, twice a product with its quantizer); the raw getter behind it takes 0.3 us"""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
 def stream():
-    return VP(torch.cuda.current_stream().cuda_stream)
+    return VP(_raw_stream())
 
 
 def _dev_u8(a, device):
@@ -357,7 +363,7 @@ class Plan(object):
 
     def launch(self):
         """the records in order on the current stream, in one C loop (kt_replay)"""
-        ss = (VP * 1)(torch.cuda.current_stream().cuda_stream)
+        ss = (VP * 1)(_raw_stream())
         gpudrv.check(gpudrv.load().kt_replay(self.recs, self.n, ss, 1), "kt_replay")
 
     def launch_nodes(self):
