@@ -1,11 +1,10 @@
 /* kt_fold.hip - the producers of a product's input, fused with its int8 quantization (k_rmsfold_qT, k_fold_fwht_qT,
    k_smfold_qT tcf.cu:370-426; their numbers are those of k_rmsfold kindi.cu:350-394 and ff_* tcf.cu:218-312).
 
-   One block of 512 threads per token row and chunk of CW = 512 NM columns (whole HB blocks, grid.x of them; NM <=
-   16): thread j holds columns c0 + j + 512 k in v[k], and every output of the chunk is made in the block. Few
-   tokens: one HB block a chunk, so a row's work is spread over C / HB blocks (the reference's grid); many tokens: the
-   widest chunk (rmsfold: the whole row), so the row is read once. rmsfold's blocks each read the whole row (NF = C /
-   512 registers) for the norm, in the reference's order, as every block of the reference does:
+   Few tokens (k_fold_q8; many: k_fold_many, below): one block of 512 threads per token row and HB block (NM = HB / 512), so
+   a row's work is spread over C / HB blocks (the reference's grid): thread j holds columns c0 + j + 512 k in v[k], and every
+   output of the chunk is made in the block. rmsfold's blocks each read the whole row (NF = C / 512 registers) for the
+   norm, in the reference's order, as every block of the reference does:
      MODE 0 (rmsfold): xf = x + (r_0 + ... + r_{n-1}) (parts in order), s = 1 / sqrt((float)(S / C) + 1e-6) with S
                        the double sum of squares, xn = (xf s) w, v = sg xn;
      MODE 1 (fold):    v = sg x;
@@ -16,8 +15,8 @@
    Bit-exact with the reference:
    - S is summed in the reference's order: thread j over k in order; each 32-lane half of a wave by the xor butterfly
      16, 8, 4, 2, 1 (the reference's warp); the 16 half-wave sums by the same butterfly (its warp 0 with lanes 16 ..
-     31 zero), which every thread evaluates from LDS. sqrt and the division go through double, which rounds to the
-     correctly rounded fp32 results the reference's IEEE sqrtf and division give.
+     31 zero), which every thread evaluates from LDS. sqrt and the division are the correctly rounded fp32 ones, as the
+     reference's IEEE sqrtf and division.
    - The transform's butterflies are the reference's pairs in the reference's stage order: stages 1 .. 32 between
      lanes of a wave; stages 64, 128, 256 (between the 8 waves) as one LDS exchange after which each thread runs the
      8-point transform of its column's 8 values (the same additions in the same order) and keeps its own output;
@@ -31,6 +30,28 @@
 template <int X> __device__ __forceinline__ float kf_bfly(float v, unsigned neg){
   return __int_as_float(__float_as_int(v) ^ neg) + kf_xorf<X>(v);
 }
+/* 1 / sqrt(S / C + 1e-6) of a row: S from the 512 threads' sums in the reference's order (each 32-lane half by the xor
+   butterfly, the 16 half-wave sums by the same one, evaluated by every thread) */
+__device__ __forceinline__ float kf_norm(double acc, double* red, int j, int C){
+  acc += kf_xord<16>(acc);
+  acc += kf_xord<8>(acc);
+  acc += kf_xord<4>(acc);
+  acc += kf_xord<2>(acc);
+  acc += kf_xord<1>(acc);
+  if((j & 31) == 0) red[j >> 5] = acc;
+  __syncthreads();
+  double t[8];
+#pragma unroll
+  for(int i = 0; i < 8; ++i) t[i] = red[i] + red[i + 8];           /* offset 8 (offset 16 added zeros) */
+#pragma unroll
+  for(int i = 0; i < 4; ++i) t[i] = t[i] + t[i + 4];
+  t[0] = t[0] + t[2];
+  t[1] = t[1] + t[3];
+  const double S = t[0] + t[1];
+  const float ms = (float)(S / (double)C) + 1e-6f;
+  return 1.0f / sqrtf(ms);                                         /* both correctly rounded */
+}
+
 template <int NM>
 __device__ __forceinline__ void kf_fwht(float* v, float* sm, int j, int HB){
   const int l = j & 63;
@@ -99,24 +120,7 @@ __global__ void __launch_bounds__(512) k_fold_q8(const KtFoldArgs a){
     double acc = 0.0;
 #pragma unroll
     for(int m = 0; m < NF; ++m){ const double d = (double)xf[m]; acc += d * d; }
-    acc += kf_xord<16>(acc);
-    acc += kf_xord<8>(acc);
-    acc += kf_xord<4>(acc);
-    acc += kf_xord<2>(acc);
-    acc += kf_xord<1>(acc);
-    if((j & 31) == 0) red[j >> 5] = acc;
-    __syncthreads();
-    double t[8];
-#pragma unroll
-    for(int i = 0; i < 8; ++i) t[i] = red[i] + red[i + 8];         /* offset 8 (offset 16 added zeros) */
-#pragma unroll
-    for(int i = 0; i < 4; ++i) t[i] = t[i] + t[i + 4];
-    t[0] = t[0] + t[2];
-    t[1] = t[1] + t[3];
-    const double S = t[0] + t[1];
-    const float ms = (float)(S / (double)CF) + 1e-6f;
-    const float q = (float)sqrt((double)ms);
-    const float s = (float)(1.0 / (double)q);
+    const float s = kf_norm(acc, red, j, CF);
     float* xw = a.xw ? a.xw + (long long)n * a.ldxw : nullptr;
     float* xn = a.xn ? a.xn + (long long)n * a.ldxn : nullptr;
     const int b0 = blockIdx.x * NM;                                /* the chunk's first register of the row */
@@ -203,78 +207,228 @@ __global__ void __launch_bounds__(512) k_fold_q8(const KtFoldArgs a){
   }
 }
 
-/* rmsfold: (chunk, row) = (HB block, row) and (row, row); fold / smfold: chunks of 1 .. 16 registers */
-template __global__ void k_fold_q8<0, 1, 1>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 2>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 3>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 4>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 5>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 6>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 7>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 8>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 9>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 10>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 11>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 12>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 13>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 14>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 15>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 1, 16>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 2>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 4>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 6>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 8>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 10>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 12>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 14>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 2, 16>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 3, 3>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 4, 4>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 5, 5>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 6, 6>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 7, 7>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 8, 8>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 8, 16>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 9, 9>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 10, 10>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 11, 11>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 12, 12>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 13, 13>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 14, 14>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 15, 15>(const KtFoldArgs);
-template __global__ void k_fold_q8<0, 16, 16>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 1, 1>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 2, 2>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 3, 3>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 4, 4>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 5, 5>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 6, 6>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 7, 7>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 8, 8>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 9, 9>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 10, 10>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 11, 11>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 12, 12>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 13, 13>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 14, 14>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 15, 15>(const KtFoldArgs);
-template __global__ void k_fold_q8<1, 16, 16>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 1, 1>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 2, 2>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 3, 3>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 4, 4>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 5, 5>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 6, 6>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 7, 7>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 8, 8>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 9, 9>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 10, 10>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 11, 11>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 12, 12>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 13, 13>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 14, 14>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 15, 15>(const KtFoldArgs);
-template __global__ void k_fold_q8<2, 16, 16>(const KtFoldArgs);
+/* ------------------------------------------------------------------ many tokens
+   The same numbers with 8 consecutive columns a thread (512 a wave, up to 4096 a block): the transform's stages 1, 2, 4 are
+   between a thread's registers, 8 .. 256 between lanes, 512 and up between the waves of an HB block (one LDS exchange), each
+   the same pairs in the same stage order; a 128-column group is 16 lanes, so its maximum and sum take 4 lane steps for 8
+   columns (6 for one in the kernel above), its divisions are made once for 8, and rows are read and written 16 bytes a lane
+   where their addresses allow (vec). rmsfold: one block a row; the norm's sum is taken first in the reference's order
+   (thread j over columns j + 512 m), the row kept in LDS.
+   Both kernels are VALU bound; MI355X, 1000 tokens: smfold of 12288 columns, HB 4096, 49.7 -> 33 us, rmsfold of 4096 with
+   one part 22.4 -> 21 us. */
+#define KF_VX 1                       /* x / r rows, sg and w in 16-byte loads */
+#define KF_VO 2                       /* xw, xn, xo in 16-byte stores */
+#define KF_VQ 4                       /* the int8 rows in 8-byte stores */
+#define KF_ROW 8                      /* smfold: a block a row, its inputs taken into LDS before an output is written */
+__device__ __forceinline__ void kf_ld8(float* v, const float* p, bool vec){
+  if(vec){
+    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  } else
+#pragma unroll
+    for(int i = 0; i < 8; ++i) v[i] = p[i];
+}
+__device__ __forceinline__ void kf_st8(float* p, const float* v, bool vec){
+  if(vec){
+    *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+  } else
+#pragma unroll
+    for(int i = 0; i < 8; ++i) p[i] = v[i];
+}
+__device__ __forceinline__ void kf_stq(int8_t* p, const int* q, bool vec){
+  if(vec){
+    uint2 o;
+    o.x = (q[0] & 255) | (q[1] & 255) << 8 | (q[2] & 255) << 16 | (unsigned)q[3] << 24;
+    o.y = (q[4] & 255) | (q[5] & 255) << 8 | (q[6] & 255) << 16 | (unsigned)q[7] << 24;
+    *(uint2*)p = o;
+  } else
+#pragma unroll
+    for(int i = 0; i < 8; ++i) p[i] = (int8_t)q[i];
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(512) k_fold_many(const KtFoldArgs a, int vec){
+  extern __shared__ __attribute__((aligned(16))) float kf_lds[];    /* [2][8][64][4] exchange, then (rmsfold) the row */
+  __shared__ double red[16];
+  float4* ex = (float4*)kf_lds;
+  float* rowb = kf_lds + 4096;
+  const int j = threadIdx.x, n = blockIdx.y, l = j & 63, C = a.C, nw = a.HB >> 9;    /* nw waves an HB block: 1, 2, 8 */
+  const int w = __builtin_amdgcn_readfirstlane(j >> 6);
+  const bool vx = vec & KF_VX, vo = vec & KF_VO, vq = vec & KF_VQ;
+  float s = 1.0f;
+  if(MODE == 0){
+    const float* x = a.x + (long long)n * a.ldx;
+    const float* r = a.r + (long long)n * a.ldr;
+    double acc = 0.0;
+    for(int m0 = 0; m0 < C; m0 += 4096){                           /* 8 columns' loads together */
+      float f[8];
+#pragma unroll
+      for(int m = 0; m < 8; ++m) f[m] = m0 + 512 * m < C ? x[m0 + 512 * m + j] : 0.0f;
+      if(a.nparts > 0){
+        float rv[8];
+#pragma unroll
+        for(int m = 0; m < 8; ++m) rv[m] = m0 + 512 * m < C ? r[m0 + 512 * m + j] : 0.0f;
+        for(int p = 1; p < a.nparts; ++p)
+#pragma unroll
+          for(int m = 0; m < 8; ++m) if(m0 + 512 * m < C) rv[m] += r[(long long)p * C + m0 + 512 * m + j];
+#pragma unroll
+        for(int m = 0; m < 8; ++m) f[m] = f[m] + rv[m];
+      }
+#pragma unroll
+      for(int m = 0; m < 8; ++m)
+        if(m0 + 512 * m < C){                                      /* uniform */
+          const double d = (double)f[m];
+          acc += d * d;
+          rowb[m0 + 512 * m + j] = f[m];
+        }
+    }
+    s = kf_norm(acc, red, j, C);                                   /* its barrier covers the row too */
+  }
+  /* smfold's product for columns c .. c + 7 */
+  auto silu = [&](int c, float* f){
+    const float* pa = a.x + (long long)n * a.ldx;
+    const float* pb = a.r + (long long)n * a.ldr;
+    float fb[8];
+    if(a.rep > 1){
+      auto src = [&](int e){ const int h = e % a.hd, g = e / a.hd; return h + a.hd * (g / a.rep + a.nk * (g % a.rep)); };
+      if(a.hd % 8 == 0){                                           /* uniform: the 8 columns stay neighbours */
+        const int sc = src(c);
+        kf_ld8(f, pa + sc, vx);
+        kf_ld8(fb, pb + sc, vx);
+      } else
+#pragma unroll
+        for(int i = 0; i < 8; ++i){ const int sc = src(c + i); f[i] = pa[sc]; fb[i] = pb[sc]; }
+    } else { kf_ld8(f, pa + c, vx); kf_ld8(fb, pb + c, vx); }
+#pragma unroll
+    for(int i = 0; i < 8; ++i) f[i] = (f[i] / (1.0f + expf(-f[i]))) * fb[i];
+  };
+  const bool whole = MODE == 0 || (MODE == 2 && (vec & KF_ROW));   /* uniform */
+  if(MODE == 2 && whole){
+    for(int c = 512 * w + 8 * l; c < C; c += 4096){
+      float f[8];
+      silu(c, f);
+      kf_st8(rowb + c, f, true);
+    }
+    __syncthreads();
+  }
+  for(int c0 = whole ? 0 : blockIdx.x * 4096; c0 < (whole ? C : (int)blockIdx.x * 4096 + 1); c0 += 4096){
+    const int c = c0 + 512 * w + 8 * l;
+    const bool on = c0 + 512 * w < C;                              /* wave-uniform */
+    float v[8];
+#pragma unroll
+    for(int i = 0; i < 8; ++i) v[i] = 0.0f;
+    if(on){
+      float sg[8];
+      kf_ld8(sg, a.sg + c, vx);
+      if(MODE == 0){
+        float f[8], wv[8];
+        kf_ld8(f, rowb + c, true);
+        kf_ld8(wv, a.w + c, vx);
+        if(a.xw && a.nparts > 0) kf_st8(a.xw + (long long)n * a.ldxw + c, f, vo);
+#pragma unroll
+        for(int i = 0; i < 8; ++i) f[i] = (f[i] * s) * wv[i];
+        if(a.xn) kf_st8(a.xn + (long long)n * a.ldxn + c, f, vo);
+#pragma unroll
+        for(int i = 0; i < 8; ++i) v[i] = sg[i] * f[i];
+      } else if(MODE == 1){
+        float f[8];
+        kf_ld8(f, a.x + (long long)n * a.ldx + c, vx);
+#pragma unroll
+        for(int i = 0; i < 8; ++i) v[i] = sg[i] * f[i];
+      } else {
+        float f[8];
+        if(whole) kf_ld8(f, rowb + c, true);
+        else silu(c, f);
+#pragma unroll
+        for(int i = 0; i < 8; ++i) v[i] = sg[i] * f[i];
+      }
+#pragma unroll
+      for(int h = 1; h < 8; h <<= 1)
+#pragma unroll
+        for(int i = 0; i < 8; ++i)
+          if(!(i & h)){ const float p = v[i], q = v[i + h]; v[i] = p + q; v[i + h] = p - q; }
+#define KF_STAGE(X) { const unsigned ng = (l & X) ? 0x80000000u : 0u; \
+      _Pragma("unroll") for(int i = 0; i < 8; ++i) v[i] = kf_bfly<X>(v[i], ng); }
+      KF_STAGE(1) KF_STAGE(2) KF_STAGE(4) KF_STAGE(8) KF_STAGE(16) KF_STAGE(32)
+#undef KF_STAGE
+    }
+    if(nw > 1){                                                    /* uniform */
+      ex[w * 64 + l] = make_float4(v[0], v[1], v[2], v[3]);
+      ex[512 + w * 64 + l] = make_float4(v[4], v[5], v[6], v[7]);
+      __syncthreads();
+      if(on)
+#pragma unroll
+        for(int hf = 0; hf < 2; ++hf){
+          float A[8][4];                                           /* the column's values in waves w ^ t */
+#pragma unroll
+          for(int t = 0; t < 8; ++t)
+            if(t < 2 || nw > 2){
+              const float4 f = ex[512 * hf + ((w ^ t) & 7) * 64 + l];
+              A[t][0] = f.x; A[t][1] = f.y; A[t][2] = f.z; A[t][3] = f.w;
+            }
+#pragma unroll
+          for(int i = 0; i < 4; ++i){
+            float s1[8], s2[8];
+            s1[0] = (w & 1) ? (A[1][i] - A[0][i]) : (A[0][i] + A[1][i]);
+            if(nw > 2){
+#pragma unroll
+              for(int t = 2; t < 8; t += 2) s1[t] = (w & 1) ? (A[t ^ 1][i] - A[t][i]) : (A[t][i] + A[t ^ 1][i]);
+#pragma unroll
+              for(int t = 0; t < 8; t += 4) s2[t] = (w & 2) ? (s1[t ^ 2] - s1[t]) : (s1[t] + s1[t ^ 2]);
+              v[4 * hf + i] = (w & 4) ? (s2[4] - s2[0]) : (s2[0] + s2[4]);
+            } else v[4 * hf + i] = s1[0];
+          }
+        }
+      __syncthreads();                                             /* the next chunk writes the exchange again */
+    }
+    if(on){
+      const float sc = a.HB == 512 ? 0.044194173824159220878f : (a.HB == 1024 ? 0.03125f : 0.015625f);
+      float m = 0.0f;
+#pragma unroll
+      for(int i = 0; i < 8; ++i){
+        v[i] = v[i] * sc;
+        m = i == 0 ? fabsf(v[0]) : fmaxf(m, fabsf(v[i]));
+      }
+      if(a.xo) kf_st8(a.xo + (long long)n * a.ldxo + c, v, vo);
+      m = fmaxf(m, kf_xorf<1>(m)); m = fmaxf(m, kf_xorf<2>(m)); m = fmaxf(m, kf_xorf<4>(m)); m = fmaxf(m, kf_xorf<8>(m));
+      const float id = m != 0.0f ? 127.0f / m : 0.0f, xs = m / 127.0f;
+      const long long n0 = a.hp ? 2 * (long long)n : n;
+      const int NG = C >> 7, g = c >> 7;
+      int q[8], sum = 0;
+#pragma unroll
+      for(int i = 0; i < 8; ++i){ q[i] = __float2int_rn(v[i] * id); sum += q[i]; }
+      kf_stq(a.Q + n0 * a.ldq + c, q, vq);
+      sum += kf_xor<1>(sum); sum += kf_xor<2>(sum); sum += kf_xor<4>(sum); sum += kf_xor<8>(sum);
+      if((l & 15) == 0){ a.XS[n0 * NG + g] = xs; a.XA[n0 * NG + g] = sum; }
+      if(a.hp){                                                    /* uniform: the residual's row */
+        const float i2 = m != 0.0f ? 32258.0f / m : 0.0f;
+        int q2[8], sum2 = 0;
+#pragma unroll
+        for(int i = 0; i < 8; ++i){
+          const float r = fmaf(-(float)q[i], xs, v[i]);
+          q2[i] = max(-127, min(127, __float2int_rn(r * i2)));
+          sum2 += q2[i];
+        }
+        kf_stq(a.Q + (n0 + 1) * a.ldq + c, q2, vq);
+        sum2 += kf_xor<1>(sum2); sum2 += kf_xor<2>(sum2); sum2 += kf_xor<4>(sum2); sum2 += kf_xor<8>(sum2);
+        if((l & 15) == 0){ a.XS[(n0 + 1) * NG + g] = m / 32258.0f; a.XA[(n0 + 1) * NG + g] = sum2; }
+      }
+    }
+  }
+}
+
+/* few tokens, an HB block a chunk: rmsfold (chunk, row), fold / smfold the chunk */
+#define KF_EACH_ROW(X) X(0, 1, 1) X(0, 1, 2) X(0, 1, 3) X(0, 1, 4) X(0, 1, 5) X(0, 1, 6) X(0, 1, 7) X(0, 1, 8) X(0, 1, 9) \
+  X(0, 1, 10) X(0, 1, 11) X(0, 1, 12) X(0, 1, 13) X(0, 1, 14) X(0, 1, 15) X(0, 1, 16) X(0, 2, 2) X(0, 2, 4) X(0, 2, 6) \
+  X(0, 2, 8) X(0, 2, 10) X(0, 2, 12) X(0, 2, 14) X(0, 2, 16) X(0, 8, 8) X(0, 8, 16) \
+  X(1, 1, 1) X(1, 2, 2) X(1, 8, 8) X(2, 1, 1) X(2, 2, 2) X(2, 8, 8)
+#define KF_INST(MODE, NM, NF) template __global__ void k_fold_q8<MODE, NM, NF>(const KtFoldArgs);
+KF_EACH_ROW(KF_INST)
+#undef KF_INST
+template __global__ void k_fold_many<0>(const KtFoldArgs, int);
+template __global__ void k_fold_many<1>(const KtFoldArgs, int);
+template __global__ void k_fold_many<2>(const KtFoldArgs, int);
 
 #define KF_KEY(MODE, NM, NF) ((MODE) * 1024 + (NM) * 32 + (NF))
 #define KF_FEW 32                     /* up to this many tokens, one HB block a chunk */
@@ -288,7 +442,7 @@ static bool kf_overlap(const float* p, int ldp, const float* q, int ldq, int M, 
 }
 
 hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
-  int cw = a.HB;
+  const int cw = a.HB;
   /* rmsfold over chunks of a row: every chunk's block reads the whole row (x and the parts, for the norm) while it
      writes its own chunk of xw / xn / xo. When one of those outputs overlaps x or the parts, one block takes the row
      (each thread writes only the columns it has read), so no block can overwrite what another has still to read. */
@@ -297,83 +451,26 @@ hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
       || kf_overlap(a.xo, a.ldxo, a.x, a.ldx, M, a.C) || (np && (kf_overlap(a.xw, a.ldxw, a.r, a.ldr, M, np * a.C)
       || kf_overlap(a.xn, a.ldxn, a.r, a.ldr, M, np * a.C) || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, np * a.C))));
   if(M > KF_FEW || alias){
-    if(mode == 0) cw = a.C;
-    else for(cw = (8192 / a.HB) * a.HB; cw > a.HB && a.C % cw; cw -= a.HB) {}
+    auto al = [](const void* p, int ld, int b){ return (uintptr_t)p % b == 0 && (long long)ld * (b == 8 ? 1 : 4) % b == 0; };
+    int vec = 0;
+    if(al(a.x, a.ldx, 16) && (!a.r || al(a.r, a.ldr, 16)) && al(a.sg, 0, 16) && (!a.w || al(a.w, 0, 16))) vec |= KF_VX;
+    if((!a.xw || al(a.xw, a.ldxw, 16)) && (!a.xn || al(a.xn, a.ldxn, 16)) && (!a.xo || al(a.xo, a.ldxo, 16))) vec |= KF_VO;
+    if(al(a.Q, a.ldq, 8)) vec |= KF_VQ;
+    /* the grouped-head order reads other chunks' columns: where xo lies over an input, a block takes the row (up to 8192
+       columns, as the norm's kernel) */
+    if(mode == 2 && a.rep > 1 && a.C <= 8192 && (kf_overlap(a.xo, a.ldxo, a.x, a.ldx, M, a.C)
+       || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, a.C))) vec |= KF_ROW;
+    const bool row = mode == 0 || (vec & KF_ROW);
+    const size_t lds = 16384 + (row ? (size_t)a.C * 4 : 0);
+    const dim3 grid(row ? 1 : (a.C + 4095) / 4096, M);
+    return kt_go(mode == 0 ? k_fold_many<0> : mode == 1 ? k_fold_many<1> : k_fold_many<2>, grid, dim3(512), lds, s, a, vec);
   }
   const int nm = cw >> 9, nf = mode == 0 ? a.C >> 9 : nm;
   void (*k)(const KtFoldArgs) = nullptr;
   switch(KF_KEY(mode, nm, nf)){
-    case KF_KEY(0, 1, 1): k = k_fold_q8<0, 1, 1>; break;
-    case KF_KEY(0, 1, 2): k = k_fold_q8<0, 1, 2>; break;
-    case KF_KEY(0, 1, 3): k = k_fold_q8<0, 1, 3>; break;
-    case KF_KEY(0, 1, 4): k = k_fold_q8<0, 1, 4>; break;
-    case KF_KEY(0, 1, 5): k = k_fold_q8<0, 1, 5>; break;
-    case KF_KEY(0, 1, 6): k = k_fold_q8<0, 1, 6>; break;
-    case KF_KEY(0, 1, 7): k = k_fold_q8<0, 1, 7>; break;
-    case KF_KEY(0, 1, 8): k = k_fold_q8<0, 1, 8>; break;
-    case KF_KEY(0, 1, 9): k = k_fold_q8<0, 1, 9>; break;
-    case KF_KEY(0, 1, 10): k = k_fold_q8<0, 1, 10>; break;
-    case KF_KEY(0, 1, 11): k = k_fold_q8<0, 1, 11>; break;
-    case KF_KEY(0, 1, 12): k = k_fold_q8<0, 1, 12>; break;
-    case KF_KEY(0, 1, 13): k = k_fold_q8<0, 1, 13>; break;
-    case KF_KEY(0, 1, 14): k = k_fold_q8<0, 1, 14>; break;
-    case KF_KEY(0, 1, 15): k = k_fold_q8<0, 1, 15>; break;
-    case KF_KEY(0, 1, 16): k = k_fold_q8<0, 1, 16>; break;
-    case KF_KEY(0, 2, 2): k = k_fold_q8<0, 2, 2>; break;
-    case KF_KEY(0, 2, 4): k = k_fold_q8<0, 2, 4>; break;
-    case KF_KEY(0, 2, 6): k = k_fold_q8<0, 2, 6>; break;
-    case KF_KEY(0, 2, 8): k = k_fold_q8<0, 2, 8>; break;
-    case KF_KEY(0, 2, 10): k = k_fold_q8<0, 2, 10>; break;
-    case KF_KEY(0, 2, 12): k = k_fold_q8<0, 2, 12>; break;
-    case KF_KEY(0, 2, 14): k = k_fold_q8<0, 2, 14>; break;
-    case KF_KEY(0, 2, 16): k = k_fold_q8<0, 2, 16>; break;
-    case KF_KEY(0, 3, 3): k = k_fold_q8<0, 3, 3>; break;
-    case KF_KEY(0, 4, 4): k = k_fold_q8<0, 4, 4>; break;
-    case KF_KEY(0, 5, 5): k = k_fold_q8<0, 5, 5>; break;
-    case KF_KEY(0, 6, 6): k = k_fold_q8<0, 6, 6>; break;
-    case KF_KEY(0, 7, 7): k = k_fold_q8<0, 7, 7>; break;
-    case KF_KEY(0, 8, 8): k = k_fold_q8<0, 8, 8>; break;
-    case KF_KEY(0, 8, 16): k = k_fold_q8<0, 8, 16>; break;
-    case KF_KEY(0, 9, 9): k = k_fold_q8<0, 9, 9>; break;
-    case KF_KEY(0, 10, 10): k = k_fold_q8<0, 10, 10>; break;
-    case KF_KEY(0, 11, 11): k = k_fold_q8<0, 11, 11>; break;
-    case KF_KEY(0, 12, 12): k = k_fold_q8<0, 12, 12>; break;
-    case KF_KEY(0, 13, 13): k = k_fold_q8<0, 13, 13>; break;
-    case KF_KEY(0, 14, 14): k = k_fold_q8<0, 14, 14>; break;
-    case KF_KEY(0, 15, 15): k = k_fold_q8<0, 15, 15>; break;
-    case KF_KEY(0, 16, 16): k = k_fold_q8<0, 16, 16>; break;
-    case KF_KEY(1, 1, 1): k = k_fold_q8<1, 1, 1>; break;
-    case KF_KEY(1, 2, 2): k = k_fold_q8<1, 2, 2>; break;
-    case KF_KEY(1, 3, 3): k = k_fold_q8<1, 3, 3>; break;
-    case KF_KEY(1, 4, 4): k = k_fold_q8<1, 4, 4>; break;
-    case KF_KEY(1, 5, 5): k = k_fold_q8<1, 5, 5>; break;
-    case KF_KEY(1, 6, 6): k = k_fold_q8<1, 6, 6>; break;
-    case KF_KEY(1, 7, 7): k = k_fold_q8<1, 7, 7>; break;
-    case KF_KEY(1, 8, 8): k = k_fold_q8<1, 8, 8>; break;
-    case KF_KEY(1, 9, 9): k = k_fold_q8<1, 9, 9>; break;
-    case KF_KEY(1, 10, 10): k = k_fold_q8<1, 10, 10>; break;
-    case KF_KEY(1, 11, 11): k = k_fold_q8<1, 11, 11>; break;
-    case KF_KEY(1, 12, 12): k = k_fold_q8<1, 12, 12>; break;
-    case KF_KEY(1, 13, 13): k = k_fold_q8<1, 13, 13>; break;
-    case KF_KEY(1, 14, 14): k = k_fold_q8<1, 14, 14>; break;
-    case KF_KEY(1, 15, 15): k = k_fold_q8<1, 15, 15>; break;
-    case KF_KEY(1, 16, 16): k = k_fold_q8<1, 16, 16>; break;
-    case KF_KEY(2, 1, 1): k = k_fold_q8<2, 1, 1>; break;
-    case KF_KEY(2, 2, 2): k = k_fold_q8<2, 2, 2>; break;
-    case KF_KEY(2, 3, 3): k = k_fold_q8<2, 3, 3>; break;
-    case KF_KEY(2, 4, 4): k = k_fold_q8<2, 4, 4>; break;
-    case KF_KEY(2, 5, 5): k = k_fold_q8<2, 5, 5>; break;
-    case KF_KEY(2, 6, 6): k = k_fold_q8<2, 6, 6>; break;
-    case KF_KEY(2, 7, 7): k = k_fold_q8<2, 7, 7>; break;
-    case KF_KEY(2, 8, 8): k = k_fold_q8<2, 8, 8>; break;
-    case KF_KEY(2, 9, 9): k = k_fold_q8<2, 9, 9>; break;
-    case KF_KEY(2, 10, 10): k = k_fold_q8<2, 10, 10>; break;
-    case KF_KEY(2, 11, 11): k = k_fold_q8<2, 11, 11>; break;
-    case KF_KEY(2, 12, 12): k = k_fold_q8<2, 12, 12>; break;
-    case KF_KEY(2, 13, 13): k = k_fold_q8<2, 13, 13>; break;
-    case KF_KEY(2, 14, 14): k = k_fold_q8<2, 14, 14>; break;
-    case KF_KEY(2, 15, 15): k = k_fold_q8<2, 15, 15>; break;
-    case KF_KEY(2, 16, 16): k = k_fold_q8<2, 16, 16>; break;
+#define KF_CASE(MODE, NM, NF) case KF_KEY(MODE, NM, NF): k = k_fold_q8<MODE, NM, NF>; break;
+    KF_EACH_ROW(KF_CASE)
+#undef KF_CASE
     default: return hipErrorInvalidValue;
   }
   return kt_go(k, dim3(a.C / cw, M), dim3(512), 0, s, a);

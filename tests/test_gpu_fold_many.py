@@ -1,0 +1,84 @@
+"""The input producers' many-token kernel (more than 32 tokens, or rmsfold with an output over its input) against the
+few-token one on the same rows: 8 columns a thread instead of one changes no pair of the transform and no order of the norm,
+so every output has the same bits; odd strides and alignments take its scalar loads and stores."""
+import numpy as np
+import pytest
+import torch
+
+from kt_cases import say, dev, rng
+
+pytestmark = pytest.mark.gpu
+FEW = 32
+
+
+def _in(t, pad, shift):
+    """the rows of t in a wider buffer: row stride + pad elements, base shifted by `shift` elements"""
+    M, C = t.shape
+    buf = torch.full((M * (C + pad) + shift + 8,), float("nan") if t.dtype == torch.float32 else 7, dtype=t.dtype, device="cuda")
+    v = buf[shift:shift + M * (C + pad)].view(M, C + pad)[:, :C]
+    v.copy_(t)
+    return v
+
+
+def _act(lin, M, C, hp, pad):
+    Mq = 2 * M if hp else M
+    q = torch.zeros((Mq, C + pad), dtype=torch.int8, device="cuda")[:, :C]
+    return lin.Act(q, torch.empty((Mq, C // 128), device="cuda"),
+                   torch.empty((Mq, C // 128), dtype=torch.int32, device="cuda"), M, C, False, hp)
+
+
+def _same(a, b):
+    return torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+# HB 512 (a wave), 1024 (two), 4096 (eight); widths of one wave, of a partial last 4096-column chunk, of many chunks
+@pytest.mark.parametrize("C,HB", [(512, 512), (1536, 512), (1024, 1024), (5120, 1024), (6144, 1024), (4096, 4096), (8192, 4096)])
+@pytest.mark.parametrize("hp", [False, True])
+@pytest.mark.parametrize("pad,shift", [(0, 0), (4, 4), (1, 3)])
+def test_many_equals_few(C, HB, hp, pad, shift):
+    from kindi_amd import linear as lin
+    M, nparts = 37, 2
+    say("fold many", C, HB, hp, pad, shift)
+    r = rng(C + HB + pad)
+    x = _in(dev(r.standard_normal((M, C)).astype(np.float32)), pad, shift)
+    b = _in(dev(r.standard_normal((M, C)).astype(np.float32)), pad, shift)
+    x[3] = 0.0
+    x[4, :128] *= 1e-30
+    parts = dev(r.standard_normal((M, nparts * C)).astype(np.float32))
+    w = _in(dev((1 + 0.2 * r.standard_normal((1, C))).astype(np.float32)), 0, shift)[0]
+    sg = _in(dev(np.where(r.random((1, C)) < 0.5, -1, 1).astype(np.float32)), 0, shift)[0]
+    perm = (C // 512, 128, 4) if C % 1024 else (24, C // 48, 2) if C % 48 == 0 else (C // 64, 32, 2)
+
+    def run(rows, order):
+        o = [_in(torch.zeros((rows.stop - rows.start, C), device="cuda"), pad, shift) for _ in range(5)]
+        acts = [_act(lin, rows.stop - rows.start, C, hp, pad) for _ in range(3)]
+        lin.rmsfold(x[rows], w, sg, HB, r=parts[rows], nparts=nparts, xw=o[0], xn=o[1], xo=o[2], out=acts[0], hp=hp)
+        lin.fold(x[rows], sg, HB, xo=o[3], out=acts[1], hp=hp)
+        lin.smfold(x[rows], b[rows], sg, HB, perm=order, xo=o[4], out=acts[2], hp=hp)
+        return o + [t for a in acts for t in (a.XQ, a.XS, a.XA)]
+
+    for order in ((1, 1, 1), perm):
+        many = run(slice(0, M), order)
+        few = [run(slice(i, min(i + FEW, M)), order) for i in range(0, M, FEW)]
+        for k, t in enumerate(many):
+            assert _same(t, torch.cat([f[k] for f in few])), (k, order)
+
+
+def test_outputs_over_inputs():
+    """rmsfold's outputs over x (any token count), smfold's xo over a in the grouped-head order (one block a row)"""
+    from kindi_amd import linear as lin
+    M, C = 40, 6144
+    r = rng(9)
+    x, b = (dev(r.standard_normal((M, C)).astype(np.float32)) for _ in range(2))
+    w, sg = torch.ones(C, device="cuda"), dev(np.where(r.random(C) < 0.5, -1, 1).astype(np.float32))
+    for m in (1, M):
+        out = [torch.empty((m, C), device="cuda") for _ in range(3)]
+        a0 = lin.rmsfold(x[:m], w, sg, 1024, r=b[:m], nparts=1, xw=out[0], xn=out[1], xo=out[2])
+        y = x[:m].clone()
+        a1 = lin.rmsfold(y, w, sg, 1024, r=b[:m], nparts=1, xo=y)
+        assert _same(y, out[2]) and _same(a0.XQ, a1.XQ) and _same(a0.XS, a1.XS)
+    want = torch.empty_like(x)
+    a0 = lin.smfold(x, b, sg, 1024, perm=(128, 24, 2), xo=want)
+    y = x.clone()
+    a1 = lin.smfold(y, b, sg, 1024, perm=(128, 24, 2), xo=y)
+    assert _same(y, want) and _same(a0.XQ, a1.XQ)
