@@ -39,7 +39,7 @@ template <bool HP> __global__ void k_quant_tern(const float*, int, int, int, int
 template <int NR> __global__ void k_quant_row(const float*, int, int, int8_t*, int, float*, int*);
 extern "C" __global__ void k_quant_q8(const float*, int, int, int, int8_t*, int, float*, int);
 extern "C" __global__ void k_tern_sum(const float*, float*, int, int, int);
-template <bool RS, bool DBG>
+template <int NW, bool RS, bool DBG>
 __global__ void k_tern_gemm_ks(const uint32_t*, const uint16_t*, int, int, const int8_t*, int, const float*, int, float*,
                                uint16_t*, int, int32_t*, int, int);
 template <int T, bool RS, bool DBG>
@@ -579,7 +579,10 @@ int kt_tern_sum(const float* P, float* y, int R, int M, int sp, void* stream){
 /* ------------------------------------------------------------------ prefill product */
 /* Which kernel, by how many 32 x 32 output tiles the launch has (every one runs the same per-element chain, so the bits
    do not depend on the choice; MI355X, 256 CUs, group scales):
-   - up to 2 a CU: k_tern_gemm_ks, a tile a block with its groups dealt over 4 waves (two such blocks share a CU):
+   - up to one a CU and rows of 4096 columns or more: k_tern_gemm_ks<8>, a tile a block with its groups dealt over 8 waves (a
+     block fills a CU's LDS): [4096 x 12288] at 61 tokens 18.1 against 20.7 us for 4 waves, [4096 x 4096] 8.7 against 9.2,
+     but [2048 x 2048] 5.6 against 5.3;
+   - up to 2 a CU: k_tern_gemm_ks<4> (two such blocks share a CU):
      [5120 x 5120] at 61 / 96 tokens (320 / 480 tiles) 13.0 / 13.7 against 18.6 / 19.0 us for k_tern_gemm_w<1>, [4096 x
      12288] at 128 (512) 28 against 40; past it [5120 x 5120] at 128 (640) 19.9 against 19.1, [17408 x 5120] at 61
      (1088) 30 against 24;
@@ -605,16 +608,15 @@ int kt_tern_gemm(const void* W, int R, int C, const int8_t* XQ, int ldq, const f
   if(ec) return ec;
   const long long rt = (R + 31) / 32, tt = (M + 31) / 32, tiles = rt * tt;
   const int gx = (R + 127) / 128;
-#define KT_PF(K, GX, GY) KT_LAUNCH((K), dim3((unsigned)((GX) * (GY))), dim3(256), 0, s, codes, scales, R, NG, XQ, ldq, XS, \
+#define KT_PF(NT, K, GX, GY) KT_LAUNCH((K), dim3((unsigned)((GX) * (GY))), dim3(NT), 0, s, codes, scales, R, NG, XQ, ldq, XS, \
                                    M, Y, Y16, ldy, dbg, (int)(GX), (int)(GY))
-#define KT_PFS(K, GX, GY, ...) do { \
-    if(per_row){ if(dbg) KT_PF((K<__VA_ARGS__ true, true>), GX, GY); else KT_PF((K<__VA_ARGS__ true, false>), GX, GY); } \
-    else { if(dbg) KT_PF((K<__VA_ARGS__ false, true>), GX, GY); else KT_PF((K<__VA_ARGS__ false, false>), GX, GY); } } while(0)
-#define KT_COMMA ,
-  if(tiles <= 2ll * cus) KT_PFS(k_tern_gemm_ks, rt, tt, );
-  else if(gx * tt <= 3ll * cus) KT_PFS(k_tern_gemm_w, gx, tt, 1 KT_COMMA);
-  else KT_PFS(k_tern_gemm_w, gx, (M + 63) / 64, 2 KT_COMMA);
-#undef KT_COMMA
+#define KT_PFS(NT, K, V, GX, GY) do { \
+    if(per_row){ if(dbg) KT_PF(NT, (K<V, true, true>), GX, GY); else KT_PF(NT, (K<V, true, false>), GX, GY); } \
+    else { if(dbg) KT_PF(NT, (K<V, false, true>), GX, GY); else KT_PF(NT, (K<V, false, false>), GX, GY); } } while(0)
+  if(tiles <= cus && NG >= 32) KT_PFS(512, k_tern_gemm_ks, 8, rt, tt);
+  else if(tiles <= 2ll * cus) KT_PFS(256, k_tern_gemm_ks, 4, rt, tt);
+  else if(gx * tt <= 3ll * cus) KT_PFS(256, k_tern_gemm_w, 1, gx, tt);
+  else KT_PFS(256, k_tern_gemm_w, 2, gx, (M + 63) / 64);
 #undef KT_PFS
 #undef KT_PF
   return 0;

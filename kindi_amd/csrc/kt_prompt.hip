@@ -4,10 +4,9 @@
    The numbers are k_tern_gemm_w's (kt_prefill.hip): Y[t][r] = sum_g fmaf((float)v(t, r, g), XS[t][g] * d[r][g], .) over
    the 128-column groups g in order (RS: fmaf(v, d, .), times XS[t][0] at the end), v the exact int32 of
    V_MFMA_I32_32X32X32_I8. The chain over g is serial by that definition, the values v are not: a block owns one tile of
-   32 tokens x 32 weight rows and its 4 waves take the groups in turn (wave w of round j: group 4 j + w). A wave makes its
+   32 tokens x 32 weight rows and its NW = 4 or 8 waves take the groups in turn (wave w of round j: group NW j + w). A wave makes its
    group's values with the packed trits unpacked in registers and hands them over through LDS as floats (exact: |v| <=
-   128 * 127); after one barrier a round every thread applies the round's 4 groups, in order, to its own 4 outputs
-   (register quad w of the tile).
+   128 * 127); after one barrier a round every thread applies the round's NW groups, in order, to its own 16 / NW outputs.
 
    Every global read is a DMA to LDS (kt_dma.h), counted by hand: a wave's own stage of a round holds its group's
    activations (4 KB, 16-byte chunk c of row r at position c ^ ((r >> 1) & 7): no bank conflicts), packed trits (1 KB),
@@ -27,12 +26,13 @@ typedef int kt_v16i __attribute__((ext_vector_type(16)));
 #define KS_STAGE (KS_D + 256)         /* token scales: 32 floats (256 bytes written) */
 #define KS_NS 3
 
-template <bool RS, bool DBG>
-__global__ void __launch_bounds__(256) k_tern_gemm_ks(const uint32_t* __restrict__ codes,
+template <int NW, bool RS, bool DBG>
+__global__ void __launch_bounds__(64 * NW) k_tern_gemm_ks(const uint32_t* __restrict__ codes,
     const uint16_t* __restrict__ scales, int R, int NG, const int8_t* __restrict__ XQ, int ldq,
     const float* __restrict__ XS, int M, float* __restrict__ Y, uint16_t* __restrict__ Y16, int ldy,
     int32_t* __restrict__ dbg, int gx, int gy){
-  __shared__ __attribute__((aligned(16))) uint8_t lds[KS_NS][4][KS_STAGE];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[KS_NS][NW][KS_STAGE];
+  constexpr int EPT = 16 / NW;                                     /* outputs a thread: 4 or 2 */
   constexpr int DMA = RS ? 6 : 7;                                  /* a wave's DMA instructions a round */
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, n = lane & 31, lr8 = lane >> 3, R8 = kt_r8(R);
@@ -59,21 +59,24 @@ __global__ void __launch_bounds__(256) k_tern_gemm_ks(const uint32_t* __restrict
   const int srg = (r0 >> 3) + (lane >> 2);
   const uint32_t ho = lane < 16 && srg < R8 ? (uint32_t)srg * (uint32_t)NG * 16u + (lane & 3) * 4 : OOB;
   const uint32_t so = lane < 32 && n0 + lane < M ? (uint32_t)(n0 + lane) * (uint32_t)NG * 4u : OOB;
-  const int rounds = (NG + 3) >> 2;
+  const int rounds = (NG + NW - 1) / NW;
   /* round j's group into stage q (past the last group it is read again: a wave's counts stay the same) */
   auto issue = [&](int j, int q){
-    const int g = min(4 * j + w, NG - 1), nc = min(8, NG - (g & ~7));
-    const uint32_t st = lbase + (uint32_t)(q * 4 * KS_STAGE);
+    const int g = min(NW * j + w, NG - 1), nc = min(8, NG - (g & ~7));
+    const uint32_t st = lbase + (uint32_t)(q * NW * KS_STAGE);
 #pragma unroll
     for(int i = 0; i < 4; ++i) kt_dma16(rx, xo[i], g * 128, st + i * 1024);
     kt_dma16(rw, wo + (uint32_t)(h * (nc * 128)), (g >> 3) * 2048 + (g & 7) * 128, st + KS_A);
     kt_dma4(rh, ho, g * 16, st + KS_B);
     if(!RS) kt_dma4(rs, so, g * 4, st + KS_D);
   };
+  const int tok0 = 8 * (EPT * w / 4) + 4 * h + EPT * w % 4;        /* this thread's outputs: tokens tok0 .. of row n */
   int aoff[4];
 #pragma unroll
   for(int i = 0; i < 4; ++i) aoff[i] = n * 128 + (((4 * h + i) ^ ((n >> 1) & 7)) << 4);
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  float acc[EPT];
+#pragma unroll
+  for(int e = 0; e < EPT; ++e) acc[e] = 0.0f;
 
   /* round j's values into stage q: this wave's DMAs of round j have landed when at most round j + 1's are in flight
      (loads retire in order) */
@@ -101,7 +104,7 @@ __global__ void __launch_bounds__(256) k_tern_gemm_ks(const uint32_t* __restrict
       *(float4*)(st + (64 * i + lane) * 16) = make_float4((float)c[4 * i], (float)c[4 * i + 1], (float)c[4 * i + 2],
                                                           (float)c[4 * i + 3]);
     if(DBG){
-      const int g = 4 * j + w;
+      const int g = NW * j + w;
       if(g < NG && row < R)
 #pragma unroll
         for(int e = 0; e < 16; ++e){
@@ -114,25 +117,25 @@ __global__ void __launch_bounds__(256) k_tern_gemm_ks(const uint32_t* __restrict
      applied in order to this thread's outputs (tokens 8 w + 4 h .. + 3, row n) while the next round's values are made */
   auto round = [&](int j, int q){
     __syncthreads();
-    float4 v[4], s[4];
-    uint16_t hd[4];
+    float v[NW][EPT], s[NW][EPT];
+    uint16_t hd[NW];
 #pragma unroll
-    for(int k = 0; k < 4; ++k){
+    for(int k = 0; k < NW; ++k){
       const uint8_t* sk = lds[q][k];
-      v[k] = *(const float4*)(sk + (64 * w + lane) * 16);
-      if(!RS) s[k] = *(const float4*)(sk + KS_D + 32 * w + 16 * h);
+      const float* pv = (const float*)(sk + (64 * (EPT * w / 4) + lane) * 16 + (EPT * w % 4) * 4);
+      const float* ps = (const float*)(sk + KS_D) + tok0;
+#pragma unroll
+      for(int e = 0; e < EPT; ++e){ v[k][e] = pv[e]; s[k][e] = RS ? 1.0f : ps[e]; }
       hd[k] = *(const uint16_t*)(sk + KS_B + 2 * n);
     }
     if(j > 0 && j + 2 < rounds) issue(j + 2, (q + 2) % KS_NS);
     if(j + 1 < rounds) make(j + 1, (q + 1) % KS_NS);
 #pragma unroll
-    for(int k = 0; k < 4; ++k)
-      if(4 * j + k < NG){                                          /* uniform */
+    for(int k = 0; k < NW; ++k)
+      if(NW * j + k < NG){                                         /* uniform */
         const float d = kt_h2f(hd[k]);
-        acc[0] = fmaf(v[k].x, RS ? d : s[k].x * d, acc[0]);
-        acc[1] = fmaf(v[k].y, RS ? d : s[k].y * d, acc[1]);
-        acc[2] = fmaf(v[k].z, RS ? d : s[k].z * d, acc[2]);
-        acc[3] = fmaf(v[k].w, RS ? d : s[k].w * d, acc[3]);
+#pragma unroll
+        for(int e = 0; e < EPT; ++e) acc[e] = fmaf(v[k][e], RS ? d : s[k][e] * d, acc[e]);
       }
   };
 #pragma unroll
@@ -146,8 +149,8 @@ __global__ void __launch_bounds__(256) k_tern_gemm_ks(const uint32_t* __restrict
   for(int q = 0; q < KS_NS - 1; ++q) if(j + q < rounds) round(j + q, q);
   const __amdgpu_buffer_rsrc_t rsx = __builtin_amdgcn_make_buffer_rsrc((void*)XS, (short)0, M * NG * 4, 0x00020000);
 #pragma unroll
-  for(int e = 0; e < 4; ++e){
-    const int t = n0 + 8 * w + 4 * h + e;
+  for(int e = 0; e < EPT; ++e){
+    const int t = n0 + tok0 + e;
     if(t < M && row < R){
       float y = acc[e];
       if(RS) y *= __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsx, (uint32_t)t * NG * 4, 0, 0));
@@ -158,6 +161,7 @@ __global__ void __launch_bounds__(256) k_tern_gemm_ks(const uint32_t* __restrict
   }
 }
 
-#define KT_KS(RS, DBG) template __global__ void k_tern_gemm_ks<RS, DBG>(const uint32_t*, const uint16_t*, int, int, \
+#define KT_KS(NW, RS, DBG) template __global__ void k_tern_gemm_ks<NW, RS, DBG>(const uint32_t*, const uint16_t*, int, int, \
     const int8_t*, int, const float*, int, float*, uint16_t*, int, int32_t*, int, int);
-KT_KS(false, false) KT_KS(false, true) KT_KS(true, false) KT_KS(true, true)
+KT_KS(4, false, false) KT_KS(4, false, true) KT_KS(4, true, false) KT_KS(4, true, true)
+KT_KS(8, false, false) KT_KS(8, false, true) KT_KS(8, true, false) KT_KS(8, true, true)

@@ -1,5 +1,5 @@
 """The prefill product's kernels at the edges of their dispatch (kt_tern_gemm): a tile a block with its groups dealt over
-4 waves (up to 2 tiles of 32 x 32 a CU), one tile a wave (up to 12), two tiles a wave. Every one applies the reference
+4 or (one tile a CU, 4096 columns or more) 8 waves (up to 2 tiles of 32 x 32 a CU), one tile a wave (up to 12), two tiles a wave. Every one applies the reference
 expression group after group, so the int32 group values and the fp32 outputs are the oracle's, bit for bit."""
 import numpy as np
 import pytest
@@ -26,6 +26,7 @@ def _route(R, M):
 @pytest.mark.parametrize("R,C,M,route", [
     (8, 128, 1, "split"), (40, 256, 17, "split"), (100, 384, 33, "split"), (31, 512, 64, "split"), (65, 640, 31, "split"),
     (257, 1152, 45, "split"), (96, 1664, 96, "split"), (5120, 1408, 61, "split"),
+    (40, 4096, 33, "split"), (31, 4224, 64, "split"), (257, 5248, 17, "split"), (1024, 6016, 70, "split"),
     (8200, 128, 70, "one"), (8200, 256, 95, "one"), (8193, 384, 65, "one"), (8260, 512, 100, "one"), (8300, 1152, 97, "one"),
     (8200, 128, 400, "two"), (8197, 256, 385, "two"), (8200, 384, 449, "two"), (8300, 1280, 390, "two")])
 @pytest.mark.parametrize("per_row", [False, True])
