@@ -283,9 +283,16 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
   float* xsl = (float*)(kt_lds + (size_t)KS * KQ * NT * 32 * 4) + (size_t)wvi * 512;
   int* xal = (int*)(xsl + 256);
   /* activations through a buffer resource over the M token rows (lanes past the pass's tokens: past the range,
-     zeros without a memory access) */
+     zeros without a memory access). A load has 4 neighbouring lanes on one row: in the operand's own order (16 lanes on 16
+     rows) it holds the address unit 27.5 ns, so 7.2 (measured a CU): MI355X, 16 tokens, 27B gate/up 25.6 -> 20.4 us, down 17.5 -> 15.0,
+     q/k/v 8.0 -> 7.3, o 7.2 -> 6.6, with the token scales' loads regrouped the same way. The rows then go through this wave's slot of red (2 KB,
+     its slice sums' place, free until they are written) into the operand order: row r of 128 bytes, 16-byte chunk c at
+     position c ^ f(r), f the bits of (r >> 1) & 7 rotated so that neither the 4-row writes nor the 16-row reads share banks */
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)xq, (short)0, a.M * a.ldq, 0x00020000);
-  const uint32_t xoff = n < nt ? (uint32_t)((t0 + n) * a.ldq + 16 * g) : (1u << 30);
+  const int lt = lane >> 2;
+  const uint32_t xoff = lt < nt ? (uint32_t)((t0 + lt) * a.ldq + 16 * (lane & 3)) : (1u << 30);
+  auto km_f = [](int r){ const int s3 = (r >> 1) & 7; return (s3 & 1) << 2 | s3 >> 1; };
+  const int awr = lt * 128 + (((lane & 3) ^ km_f(lt)) << 4), ard = n * 128 + ((g ^ km_f(n)) << 4);
   for(int it = 0, ks = sg; MS ? ks < KS : it < 1; ++it, ks += G){                /* !MS: one slice a wave */
   const int s_lo = ks * S / KS, ns = (ks + 1) * S / KS - s_lo;   /* this slice's steps (1 or 2) */
   /* entry (j 8 + c) 16 + token of the region: KQ = 1 stages the slice's 16 units, KQ = 4 only its own 4 (k-lanes cb,
@@ -296,7 +303,7 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
   int xdst[NI];
 #pragma unroll
   for(int i = 0; i < NI; ++i){
-    const int idx = lane + 64 * i, un = idx >> 4, tl = idx & 15;
+    const int idx = lane + 64 * i, un = idx % (2 * CW), tl = idx / (2 * CW);
     const int j = un / CW, c = cb + un % CW;                     /* the wave's units: CW k-lanes, 2 steps */
     const int u = (s_lo + j) * KT_KL + c;
     const int t = t0 + tl < a.M ? t0 + tl : t0;
@@ -359,8 +366,11 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
         unsigned w0 = wq[j][cc].x, w1 = wq[j][cc].y, w2 = wq[j][cc].z, w3 = wq[j][cc].w;
         km_swap32(w0, w2); km_swap32(w1, w3);
         km_swap16(w0, w1); km_swap16(w2, w3);
-        const kt_v4i A0 = {(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w};
-        const kt_v4i A1 = {(int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+        uint8_t* ab = kt_lds + (size_t)(ks * KQ + q) * 2048;       /* chunks 0 - 3 of half 0, 4 - 7 of half 1 */
+        *(kt_v4i*)(ab + awr) = kt_v4i{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w};
+        *(kt_v4i*)(ab + (awr ^ 64)) = kt_v4i{(int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+        kt_wave_sync();
+        const kt_v4i A0 = *(const kt_v4i*)(ab + ard), A1 = *(const kt_v4i*)(ab + (ard ^ 64));
         /* both chains start from -XA of tokens 4 g .. + 3 (staged negated), so they end at v = sum d q - XA */
         const int4 xa4 = *(const int4*)(xal + (j * 8 + c) * 16 + 4 * g);
         const kt_v4i cx = {xa4.x, xa4.y, xa4.z, xa4.w};
@@ -405,6 +415,7 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
   KT_M16TS(2);
   /* slices in order (KQ = 4: the pair sums of a slice first, (p0 + p1) + (p2 + p3)) */
   /* a lane's 8 sums as two float4 at [slice][quarter][half][lane]: 16-byte LDS accesses, conflict free */
+  kt_wave_sync();                                                /* the slot's last activations are read */
   {
     float4* r4 = (float4*)red + (size_t)(ks * KQ + q) * 128 + lane;
     r4[0] = make_float4(part[0], part[1], part[2], part[3]);
