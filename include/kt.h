@@ -139,7 +139,7 @@ int kt_replay(const kt_launch* recs, int n, void* const* streams, int nstreams);
    and not read (the matrix cores take signed trits). per_row = 0: Y = sum_g fmaf(v, XS[t][g] d[r][g], .) in group
    order (the reference's expression). per_row = 1 (XS from kt_quant_q8 per_row: one scale a token): Y = XS[t][0] *
    sum_g fmaf(v, d[r][g], .) in group order (two VALU operations an element and group instead of three; the same
-   bits whichever of the two block shapes R selects, within the 1e-3 tolerance of the reference's expression).
+   bits whichever kernel the sizes select, within the 1e-3 tolerance of the reference's expression).
    M ldq, M C / 32 and the packed codes stay below 2^31 bytes. Replaces k_tc_mm2 / k_tc_mm{4,8,16}
    (tc_hip.cu:243-269, chunk.py:273-296) and k_mm_g5q (chunk.cu:858-918, chunk.py:245-271). */
 int kt_tern_gemm(const void* W, int R, int C, const int8_t* XQ, int ldq, const float* XS, const int32_t* XA,

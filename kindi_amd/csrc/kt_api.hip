@@ -653,7 +653,7 @@ int kt_tern_gemm8(const int8_t* W8, const void* W, int R, int C, const int8_t* X
   const bool aligned = ldy % 8 == 0 && (!Y || kt_al(Y, 16)) && (!Y16 || kt_al(Y16, 16));   /* 16-byte output rows */
 #ifndef KT_G8_MIN_PCT
 #define KT_G8_MIN_PCT 70              /* tiles a CU, percent (measured on MI355X: gate/up [12288 x 4096] at 512 tokens,
-                                         192 tiles on 256 CUs, 53.7 -> 41.9 us over the packed-trit kernel) */
+                                         192 tiles on 256 CUs, 46 us on the packed trits, 41.9 here) */
 #endif
   if((long long)((kt_r8(R) * KT_RG + 255) / 256) * ((M + 127) / 128) * 100 < (long long)cus * KT_G8_MIN_PCT || !aligned)
     return kt_tern_gemm(W, R, C, XQ, ldq, XS, nullptr, 1, M, Y, Y16, ldy, dbg, stream);

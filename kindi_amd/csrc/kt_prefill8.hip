@@ -3,7 +3,7 @@
    k_tern_expand writes the signed trits t = d - 1 of a kt2 matrix as int8 in natural order, W8 [8 R8][C] (rows padded
    to the kt2 row groups). The product then has nothing to unpack: both operands reach LDS by DMA
    (buffer_load_dwordx4 ... lds: no registers, no LDS store instructions), and the waves only read LDS, run the
-   matrix cores and the per-group epilogue. The numbers are those of k_tern_gemm with per-row activation scales:
+   matrix cores and the per-group epilogue. The numbers are those of kt_tern_gemm with per-row activation scales:
      Y[t][r] = XS[t] * sum_g fmaf((float)v(t, r, g), d[r][g], .)      (groups in order)
    with v(t, r, g) the exact int32 group value (k_mm_g5q's int8 trits, chunk.cu:836-918; the reference expression's
    per-group value, tc_hip.cu:171).
@@ -21,9 +21,9 @@
    overlaps an MFMA only when it sits behind it in the stream). One block a CU (its 145 KB of LDS) takes tiles
    blockIdx.x, + gridDim.x, ...; a tile's outputs go out through LDS as 16-byte token rows before the next tile's
    first DMAs.
-   Measured on MI355X (config 2, M = 2048, fp16 out, against k_tern_gemm on the packed trits): gate/up [12288 x 4096]
-   131 against 199 us, down [4096 x 12288] 128 against 172 us (with two-byte stores straight from the accumulators:
-   175 and 142 us). Below one block a CU (M = 512) the packed-trit kernels are faster and kt_tern_gemm8 runs them. */
+   Measured on MI355X (config 2, M = 2048, fp16 out): gate/up [12288 x 4096] 118 .. 131 us against 138 for k_tern_gemm_w on the
+   packed trits, down [4096 x 12288] 118 .. 128 us (with two-byte stores straight from the accumulators: 175 and 142 us).
+   Below 0.7 tiles a CU kt_tern_gemm8 runs the packed-trit kernels. */
 #include "kt_common.h"
 #include "kt_dma.h"
 
