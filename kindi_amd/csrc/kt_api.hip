@@ -111,6 +111,7 @@ static bool kt_q8_gemm_takes(int NU){ return kt_steps(NU) <= KT_SL * kt_kslices(
 #endif
 #define KT_MMA_MAX 32
 #define KT_Q8_MMA_KS 8                 /* q8_0 matrix-core product: K slices a block (kt_mma.hip KM_Q8_KS) */
+#define KT_Q8_MMA_ACT (16 * 512)       /* ... and its activations in LDS, bytes a wave (kt_mma.hip KM_Q8_ACT) */
 #ifndef KT_MMA_W2
 #define KT_MMA_W2 (1ll << 26)          /* 2 tokens: the matrix cores from this many weights a launch */
 #endif
@@ -747,7 +748,7 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
        lane): [4096 x 2688] at 50 tokens 18.7 -> 12.6 us, [1024 x 1024] at 128 25.4 -> 7.5; two a CU was no faster */
     const int want = (cus + tiles - 1) / tiles, gy = want < np ? want : np;
     const dim3 grid(tiles, gy), block(64 * ks);
-    const size_t lds = (size_t)ks * 16 * 32 * 4 + (size_t)ks * 256 * 4;          /* slice sums, D */
+    const size_t lds = (size_t)ks * (16 * 32 * 4 + 256 * 4) + (size_t)ks * KT_Q8_MMA_ACT;   /* slice sums, D, activations */
     if(dbg) KT_LAUNCH((k_q8_mma<false, true, false>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
     else KT_LAUNCH((k_q8_mma<false, false, false>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
     return 0;
@@ -845,7 +846,7 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
     /* 4 or more entries an active expert on average: the matrix-core product per (32-row tile, active expert), the
        expert's whole list in passes of 16 (the same numbers and tree) */
     const dim3 grid((kt_r8(R) + 3) / 4, ny), block(64 * ks);
-    const size_t lds = (size_t)ks * 16 * 32 * 4 + (size_t)ks * 256 * 4;          /* slice sums, D */
+    const size_t lds = (size_t)ks * (16 * 32 * 4 + 256 * 4) + (size_t)(ks > 2 ? 2 : ks) * KT_Q8_MMA_ACT;   /* as above */
     const KtGemvArgs da = {};
     if(ks > 2){
       /* two waves a block taking the slices in turn (the same slice sums in the same order): blocks of 2 waves at

@@ -478,6 +478,7 @@ KM16_INST(false, 4, true) KM16_INST(true, 4, true) KM16_INST(false, 2, true) KM1
    weights again every pass. Epilogue as k_gemv_flat: per k-lane c the chain fmaf((float)v, d * D[t][u], .) over the slice's
    units 8 s + c, the butterfly's tree over c, the slices in order. */
 #define KM_Q8_KS 8                    /* at most 8 K slices (q8_0 C <= 4096): 256 VGPRs a lane */
+#define KM_Q8_ACT (KM_TOK * 512)      /* LDS bytes a wave: a pass's activations of a slice */
 template <bool GRP, bool DBG, bool MS>   /* MS: wave w takes slices w, w + W, ... (W waves a block) */
 __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, const KtGroupedArgs ga,
                                                           const int8_t* __restrict__ xq, const float* __restrict__ xd,
@@ -521,41 +522,47 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
   const int nrows = GRP ? ga.nrows : cntM;
 
   /* a pass's loads, all unconditional (clamped) and issued together: the D scales of the slice's 16 units x 16
-     tokens (to this wave's LDS region before the products, so the epilogue reads them there), and this lane's
-     activations of the 16 units through a buffer resource over the input rows (lanes past the pass's tokens read at
-     2^31, past the range, which gives zeros without a memory access; the launcher keeps the rows below 2^31 bytes) */
+     tokens (to this wave's LDS region before the products, so the epilogue reads them there), and the activations
+     of the 16 units through a buffer resource over the input rows (a token past the pass and a unit past the slice or
+     the matrix read at 2^31, past the range, which gives zeros without a memory access; the launcher keeps the rows
+     below 2^31 bytes). Neighbouring lanes are on one row: in the matrix cores' operand order (32 lanes on 16 rows) a load
+     holds the address unit 27.5 ns, so 7.2 (measured a CU). The rows go through LDS: 512 bytes each, 16-byte chunk c of
+     row r at c ^ f(r), f the two bit pairs of r exchanged (neither the 4-row writes nor the 16-row reads share banks). MI355X,
+     dense [8192 x 4096] at 16 / 50 / 100 tokens 13.2 / 25.0 / 40.4 -> 11.5 / 22.0 / 32.8 us, grouped up [1856 x 2688], 128 experts, at
+     6 / 9 entries an expert 132 / 156 -> 128 / 149 */
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)xq, (short)0, nrows * ldq, 0x00020000);
   float* xsl = (float*)(kt_lds + (size_t)KS * NT * 32 * 4) + (size_t)wv * 256;
+  uint8_t* xal = kt_lds + (size_t)KS * (NT * 32 * 4 + 256 * 4) + (size_t)wv * KM_Q8_ACT;
+  const int at = lane >> 2, ac = lane & 3, r16 = lane & 15;      /* the load's row and chunk; the operand's row */
+  const int aw = at * 512 + ((ac ^ (at >> 2)) << 4), ax = (at & 3) << 6;
+  const int ar = r16 * 512 + ((h ^ ((r16 & 3) << 2) ^ (r16 >> 2)) << 4);
   float xsv[4];
-  uint4 xa[2 * KT_KL];
+  uint4 xa[8];
   /* the pass's input rows (the list indirection) first, the loads that need them after */
   int nrq[4], na = 0;
   auto ld_rows = [&](int t0){
     const int nt = min(NT, cntM - t0);
 #pragma unroll
     for(int q = 0; q < 4; ++q){
-      const int tl = (lane + 64 * q) & 15;
+      const int tl = (lane >> 4) + 4 * q;
       const int pt = p0 + t0 + (tl < nt ? tl : 0);
       nrq[q] = xrow ? xrow[pt] : pt;
     }
-    const int pe = p0 + t0 + (lr < nt ? lr : 0);
+    const int pe = p0 + t0 + (at < nt ? at : 0);
     na = xrow ? xrow[pe] : pe;
   };
   auto ld_pass = [&](int t0){
-    const int nt = min(NT, cntM - t0);
+    const int nt = min(NT, cntM - t0), u0 = s_lo * KT_KL, nu = min(ns * KT_KL, NU - u0);   /* the slice's units */
 #pragma unroll
     for(int q = 0; q < 4; ++q){
-      const int idx = lane + 64 * q, n = idx >> 4;
-      const int u = (s_lo + (n >> 3)) * KT_KL + (n & 7);
+      const int u = u0 + r16;
       xsv[q] = xd[(long long)nrq[q] * ldd + (u < NU ? u : 0)];
     }
-    const uint32_t xo = lr < nt ? (uint32_t)(na * ldq + 16 * h) : (1u << 31);
+    const uint32_t xo = (uint32_t)(na * ldq + u0 * 32 + ac * 16);
 #pragma unroll
-    for(int n = 0; n < 2 * KT_KL; ++n){
-      const int c = n >> 1, j = n & 1, u = (s_lo + j) * KT_KL + c;
-      const int uu = (j < ns && u < NU) ? u : 0;
-      xa[n] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xr, xo + uu * 32, 0, 0));
-    }
+    for(int i = 0; i < 8; ++i)
+      xa[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xr,
+                                 at < nt && 2 * i + (ac >> 1) < nu ? xo + i * 64 : 1u << 31, 0, 0));
   };
   /* the slice's 16 units in k-lane-major order (unconditional: a unit past the slice or the matrix reads offset 0) */
   uint4 wq[2][KT_KL];
@@ -574,8 +581,13 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
   /* the slice's products for the pass at t0 into red[ks] */
   auto compute = [&](int t0){
 #pragma unroll
-    for(int q = 0; q < 4; ++q) xsl[lane + 64 * q] = xsv[q];
+    for(int q = 0; q < 4; ++q) xsl[r16 * 16 + (lane >> 4) + 4 * q] = xsv[q];
+#pragma unroll
+    for(int i = 0; i < 8; ++i) *(uint4*)(xal + (aw ^ ax ^ (i * 64))) = xa[i];
     kt_wave_sync();
+    uint4 xn[2];
+#pragma unroll
+    for(int j = 0; j < 2; ++j) xn[j] = *(const uint4*)(xal + ar + 256 * j);
     float part[NE], t01[NE], t23[NE], t45[NE], pend[NE];
 #pragma unroll
     for(int e = 0; e < NE; ++e){ part[e] = 0.0f; t01[e] = 0.0f; t23[e] = 0.0f; t45[e] = 0.0f; pend[e] = 0.0f; }
@@ -584,11 +596,14 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
       float chain[NE];
 #pragma unroll
       for(int e = 0; e < NE; ++e) chain[e] = 0.0f;
+      const uint4 xc[2] = {xn[0], xn[1]};
+#pragma unroll
+      for(int j = 0; j < 2; ++j) if(c + 1 < KT_KL) xn[j] = *(const uint4*)(xal + (ar ^ ((c + 1) * 32)) + 256 * j);
 #pragma unroll
       for(int j = 0; j < 2; ++j){
         const int s = s_lo + j, u = s * KT_KL + c;
         const bool uok = j < ns && u < NU;                      /* wave-uniform */
-        const uint4 x = xa[2 * c + j];
+        const uint4 x = xc[j];
         if(uok){
           const float d = rok ? kt_h2f(hq[j][c]) : 0.0f;
           const kt_v4i A = {(int)x.x, (int)x.y, (int)x.z, (int)x.w};
@@ -616,6 +631,7 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
     }
 #pragma unroll
     for(int e = 0; e < NE; ++e) red[((size_t)ks * NT + km_tok(e, lane)) * 32 + lr] = part[e];
+    kt_wave_sync();                                              /* the next slice or pass overwrites xsl and xal */
   };
   /* the pass's slice sums in slice order, by wave 0 */
   auto finish = [&](int t0){
