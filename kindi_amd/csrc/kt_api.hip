@@ -724,8 +724,8 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
      - the matrix cores with a K slice a wave (k_q8_mma, up to 8 slices) from 9 tokens, from 5 on 2^22 weights, from 3 on
        2^25: [2688 x 1856] at 4 / 5 tokens 6.4 against 7.4 / 8.3 -> 7.3 us, [8192 x 4096] at 3 tokens 14.2 -> 11.5,
        [1024 x 1024] at 5 / 10 tokens 6.1 against 6.8 / 8.1 -> 6.9;
-     - k_q8_gemm above 10 (tile of 32 rows, pass of 16 tokens) pairs a CU: [4096 x 2688] at 256 / 600 tokens (2048 / 4864
-       pairs) 33 against 41 / 70 -> 52 us, [8192 x 4096] at 128 / 256 (2048 / 4096) 47 against 54 / 87 -> 56; and from 64
+     - k_q8_gemm above 12 (tile of 32 rows, pass of 16 tokens) pairs a CU: [8192 x 4096] at 176 tokens (11 pairs) 49 against 56
+       us, at 224 (14) 59 -> 56, at 288 (18) 72 -> 61; [4096 x 2688] at 336 (10.5) 41 against 42, at 448 (14) 50 -> 42; and from 64
        tokens where the rows have more than 8 slices: [4096 x 8192] at 50 / 100 tokens 117 / 217 against 98 / 99 us,
        [1024 x 5120] 42 / 76 against 63 / 63;
      - the v_dot4 kernel else. */
@@ -734,7 +734,7 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
   if(ec) return ec;
   const int tiles = (kt_r8(R) + 3) / 4, np = M / 16 + (M % 16 ? 1 : 0);
   const long long nw = (long long)R * C;
-  if((ks <= KT_Q8_MMA_KS ? (long long)tiles * np > 10ll * cus : M >= 64) && kt_q8_gemm_takes(NB)
+  if((ks <= KT_Q8_MMA_KS ? (long long)tiles * np > 12ll * cus : M >= 64) && kt_q8_gemm_takes(NB)
      && (long long)M * ldq < (1ll << 31)
      && (long long)M * ldd * 4 < (1ll << 31) && (long long)kt_r8(R) * NB * 272 < (1ll << 31) && (M + 63) / 64 <= 65535){
     const dim3 grid((R + 127) / 128, (M + 63) / 64);
@@ -823,13 +823,16 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
   const int ks = kt_kslices(a.NU);
   const int ny = E < nentries ? E : nentries;
   hipStream_t s = kt_stream(stream);
-  /* 10 or more entries an expert on average: k_q8_gemm, whose two tiles of 32 entries a wave share the weights (MI355X, 128
-     experts, 6 picks, up [1856 x 2688] / down [2688 x 1856]: at 96 entries 1003 / 976 -> 398 / 391 us, 24: 310 / 304 -> 174
-     / 179, 12: 181 / 172 -> 158 / 168, but 9: 152 / 151 against 153 / 164); from 4 where the rows have more slices than
-     k_q8_mma takes */
+  /* Entries an expert on average from which k_q8_gemm, whose two tiles of 32 entries a wave share the weights, is faster
+     (MI355X, k_q8_mma against it; router scores with a bias of 0.1 N(0, 1), as popular experts have, up [1856 x 2688] / down
+     [2688 x 1856] of 128 experts, 6 picks): 96 entries 1003 / 976 -> 398 / 391 us, 24: 310 / 304 -> 174 / 179, 12: 195 / 182 -> 146 /
+     147, 9: 170 / 152 -> 130 / 133, 7: 146 / 149 -> 131 / 134, but 5: 117 / 120 against 107 / 122 and 4: 109 against 114 down; with no
+     bias 8: 154 against 156, 6: 149 against 153. So 7; 10 where the rows have up to 2 slices ([1000 x 512] of 64 experts at 8 / 9
+     entries 18.9 / 18.8 against 19.8 / 18.7), 4 where they have more slices than k_q8_mma takes */
+  const long long many = ks <= 2 ? 10 : ks <= KT_Q8_MMA_KS ? 7 : 4;
   const bool off32 = (long long)a.nrows * ldq < (1ll << 31) && (long long)a.nrows * ldd * 4 < (1ll << 31)
                      && (long long)kt_r8(R) * a.NU * 272 < (1ll << 31);
-  if(nentries >= (ks <= KT_Q8_MMA_KS ? 10ll : 4ll) * ny && off32 && kt_q8_gemm_takes(a.NU)){
+  if(nentries >= many * ny && off32 && kt_q8_gemm_takes(a.NU)){
     /* P blocks share a row tile's passes of 64, so that a long list (a popular expert) does not hold one block's CU to the
        end: router scores with a bias of 0.1 N(0, 1), 96 entries an expert, P 1 / 3 / 7: up 678 / 471 / 427 us, 48: 360 / 287
        / 260; without the bias 396 / 385 / 392. Odd: the blocks past a list's end leave at once, and an even P left the same

@@ -28,16 +28,31 @@ LENS = [0, 1, 31, 32, 33, 64, 65, 130]
 @pytest.mark.parametrize("C", [32, 96, 256, 288, 544, 1856, 2688, 4096, 4352, 16384])
 @pytest.mark.parametrize("R", [8, 100, 129])
 def test_grouped_lists(R, C):
+    assert sum(LENS) >= 10 * len(LENS)
+    _grouped(R, C, LENS)
+
+
+# 4 to 6 entries an expert: k_q8_mma (its lists around the pass of 16; one and several slices a wave, odd counts)
+FEW = [0, 1, 3, 15, 16, 2, 17, 1]
+
+
+@gpu
+@pytest.mark.parametrize("C", [32, 96, 288, 544, 1536, 1856, 2688, 4096])
+@pytest.mark.parametrize("R", [8, 100])
+def test_grouped_few(R, C):
+    assert 4 * len(FEW) <= sum(FEW) < 7 * len(FEW)
+    _grouped(R, C, FEW)
+
+
+def _grouped(R, C, lens):
     from kindi_amd import moe
-    from kindi_amd.linear import ptr
-    say("grouped gemm", R, C)
-    E, n = len(LENS), sum(LENS)
-    assert n >= 10 * E
+    say("grouped", R, C, lens)
+    E, n = len(lens), sum(lens)
     cases = [q8_case(R, C, 1000 * R + C + e) for e in range(E)]
     W = moe.Q8Experts([c[0] for c in cases], R, C)
     M = 70                                                                # input rows, reached through xrow
     Q, D = moe.q8_quantize(dev(rng(C).normal(0, 1, (M, C)).astype(np.float32)))
-    cnt = np.array(LENS, np.int32)
+    cnt = np.array(lens, np.int32)
     off = np.concatenate([[0], np.cumsum(cnt)[:-1]]).astype(np.int32)
     act = np.concatenate([np.flatnonzero(cnt), np.zeros(1)]).astype(np.int32)
     xrow = rng(7).integers(0, M, n).astype(np.int32)
@@ -64,7 +79,7 @@ def test_grouped_lists(R, C):
 
 @gpu
 @pytest.mark.parametrize("R,C,M", [(8, 32, 3), (100, 96, 9), (2688, 1856, 5), (4096, 2688, 50), (4100, 2688, 330),
-                                   (8192, 4096, 4), (8190, 1024, 161), (130, 4352, 64), (136, 16384, 65), (136, 8192, 65), (40, 8192, 70)])
+                                   (8192, 4096, 4), (8190, 1024, 161), (4100, 2688, 400), (8190, 1024, 200), (130, 4352, 64), (136, 16384, 65), (136, 8192, 65), (40, 8192, 70)])
 def test_dense_routes(R, C, M):
     from kindi_amd import moe
     say("q8 dense", R, C, M)
