@@ -827,9 +827,9 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
      (MI355X, k_q8_mma against it; router scores with a bias of 0.1 N(0, 1), as popular experts have, up [1856 x 2688] / down
      [2688 x 1856] of 128 experts, 6 picks): 96 entries 1003 / 976 -> 398 / 391 us, 24: 310 / 304 -> 174 / 179, 12: 195 / 182 -> 146 /
      147, 9: 170 / 152 -> 130 / 133, 7: 146 / 149 -> 131 / 134, but 5: 117 / 120 against 107 / 122 and 4: 109 against 114 down; with no
-     bias 8: 154 against 156, 6: 149 against 153. So 7; 10 where the rows have up to 2 slices ([1000 x 512] of 64 experts at 8 / 9
+     bias 8: 154 against 156, 6: 149 against 153. So 8, where neither router loses; 10 where the rows have up to 2 slices ([1000 x 512] of 64 experts at 8 / 9
      entries 18.9 / 18.8 against 19.8 / 18.7), 4 where they have more slices than k_q8_mma takes */
-  const long long many = ks <= 2 ? 10 : ks <= KT_Q8_MMA_KS ? 7 : 4;
+  const long long many = ks <= 2 ? 10 : ks <= KT_Q8_MMA_KS ? 8 : 4;
   const bool off32 = (long long)a.nrows * ldq < (1ll << 31) && (long long)a.nrows * ldd * 4 < (1ll << 31)
                      && (long long)kt_r8(R) * a.NU * 272 < (1ll << 31);
   if(nentries >= many * ny && off32 && kt_q8_gemm_takes(a.NU)){
