@@ -15,8 +15,10 @@
    bytes, 16-byte chunk i of row t at i ^ (t & 15); token scales [row][16], 4-float chunk i of row t at i ^ ((t >> 2) & 3).
    A unit past the matrix or the slice gets zero scales (its product is +0).
 
-   Measured on MI355X (128 experts, 6 picks, up [1856 x 2688], against k_q8_mma): 96 entries an expert 1003 -> 398 us, 24:
-   310 -> 174 us, 12: 181 -> 158 us (678 MB of weights: 4.3 TB/s). At long lists the SIMDs bound it: a unit of a tile takes
+   Measured on MI355X (128 experts, 6 picks, even router, up [1856 x 2688] / down [2688 x 1856], against k_q8_mma): 96
+   entries an expert 1003 / 981 -> 394 / 372 us, 24: 309 / 302 -> 174 / 157, 12: 166 / 168 -> 152 / 151 (678 MB of weights: 4.5 TB/s).
+   The refill goes out only where another slice or pass of the block follows: with one after the last (KS + 1 slices read for
+   KS) 12 entries took 156 / 167 us, 24: 178 / 176. At long lists the SIMDs bound it: a unit of a tile takes
    about 37 vector and 1.5 matrix instructions, and 2 waves a SIMD (253 registers) issue at most one vector instruction
    each about every 4 cycles; without any global load 96 entries take 296 us. */
 #include <type_traits>
@@ -206,8 +208,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
         if(refilled && !DBG) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(KT_QG_LOADS) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        refilled = tt + 1 == T;
-        if(!refilled) issue(st ^ 1, tt + 1, s0, ns, nt);
+        /* the weights' last tile refills them, for the next slice or the first one of the block's next pass */
+        refilled = tt + 1 == T && (k + 1 < KS || t0 + t_st < t_hi);
+        if(tt + 1 < T) issue(st ^ 1, tt + 1, s0, ns, nt);
         else if(k + 1 < KS) issue(st ^ 1, 0, sn, nsn, nt);
         tile(refilled, st, tt, k, s0, ns, sn, nsn, t0);
         st ^= 1;

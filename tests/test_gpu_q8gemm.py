@@ -44,6 +44,37 @@ def test_grouped_few(R, C):
     _grouped(R, C, FEW)
 
 
+# lists of more than one pass a block: 64 P entries a round of the P blocks that share a row tile (P = 3 below 64 entries an
+# expert on average, 7 from there on), so second and third passes of one and two tiles, and blocks with no pass at all
+LONG3 = [0, 1, 420, 33, 2, 3, 0, 5]
+LONG3B = [193, 0, 257, 1, 0, 2, 1, 0]
+LONG7 = [0, 1, 449, 520, 64, 96, 3, 30]
+
+
+@gpu
+@pytest.mark.parametrize("lens", [LONG3, LONG3B, LONG7], ids=["three", "three_b", "seven"])
+@pytest.mark.parametrize("C", [256, 512, 1856, 2688, 4352])       # one slice, one of two steps, 4, 6 (the last short), 9 slices
+def test_grouped_passes(C, lens):
+    mean = sum(lens) // len(lens)
+    assert 12 <= mean and (mean >= 64) == (lens is LONG7) and max(lens) > 64 * (7 if mean >= 64 else 3)
+    _grouped(100, C, lens)
+
+
+def _active(cnt):
+    """the active experts in ascending order (E entries, the tail unused) and how many there are"""
+    on = np.flatnonzero(cnt)
+    act = np.zeros(len(cnt), np.int32)
+    act[:len(on)] = on
+    return act, np.array([len(on)], np.int32)
+
+
+@pytest.mark.parametrize("lens", [LENS, FEW, LONG3, LONG3B, LONG7])
+def test_lists_are_whole(lens):
+    """the lists that the tests here hand to the kernel, which trusts them: every active expert once, none past the table"""
+    act, nact = _active(np.array(lens, np.int32))
+    assert nact[0] <= len(act) == len(lens) and sorted(act[:nact[0]]) == [e for e, c in enumerate(lens) if c]
+
+
 def _grouped(R, C, lens):
     from kindi_amd import moe
     say("grouped", R, C, lens)
@@ -54,9 +85,9 @@ def _grouped(R, C, lens):
     Q, D = moe.q8_quantize(dev(rng(C).normal(0, 1, (M, C)).astype(np.float32)))
     cnt = np.array(lens, np.int32)
     off = np.concatenate([[0], np.cumsum(cnt)[:-1]]).astype(np.int32)
-    act = np.concatenate([np.flatnonzero(cnt), np.zeros(1)]).astype(np.int32)
     xrow = rng(7).integers(0, M, n).astype(np.int32)
-    lists = (dev(cnt), dev(off), dev(xrow), dev(np.zeros(n, np.int32)), dev(act), dev(np.array([E - 1], np.int32)))
+    act, nact = _active(cnt)
+    lists = (dev(cnt), dev(off), dev(xrow), dev(np.zeros(n, np.int32)), dev(act), dev(nact))
     Y = torch.full((n, R), float("nan"), device="cuda")
     dbg = torch.empty((n, R, C // 32), dtype=torch.int32, device="cuda")
     W.grouped(lists, M, Q, D, Y, dbg=dbg)
