@@ -214,8 +214,10 @@ __global__ void __launch_bounds__(512) k_fold_q8(const KtFoldArgs a){
    columns (6 for one in the kernel above), its divisions are made once for 8, and rows are read and written 16 bytes a lane
    where their addresses allow (vec). rmsfold: one block a row; the norm's sum is taken first in the reference's order
    (thread j over columns j + 512 m), the row kept in LDS.
-   Both kernels are VALU bound; MI355X, 1000 tokens: smfold of 12288 columns, HB 4096, 49.7 -> 33 us, rmsfold of 4096 with
-   one part 22.4 -> 21 us. */
+   MI355X, 1000 tokens, against the kernel above on chunks of up to 8192 columns (rmsfold: the row): smfold of 12288 columns, HB
+   4096, 45.1 -> 30.3 us, rmsfold of 4096 with one part and xw 21.3 -> 15.1, of 5120 at 33 / 256 tokens 10.2 / 11.3 -> 7.0 / 8.0.
+   waves_per_eu holds the registers to three blocks a CU for rmsfold (80; 88 and two blocks without: 57.8 against 66.5 us at
+   4096 tokens of 8192 columns) and to five waves a SIMD for smfold (3 %). */
 #define KF_VX 1                       /* x / r rows, sg and w in 16-byte loads */
 #define KF_VO 2                       /* xw, xn, xo in 16-byte stores */
 #define KF_VQ 4                       /* the int8 rows in 8-byte stores */
@@ -228,13 +230,28 @@ __device__ __forceinline__ void kf_ld8(float* v, const float* p, bool vec){
 #pragma unroll
     for(int i = 0; i < 8; ++i) v[i] = p[i];
 }
-__device__ __forceinline__ void kf_st8(float* p, const float* v, bool vec){
+/* a wave's 512 columns (lane l: 8 l .. + 7) to p, through t, 512 floats of LDS of the wave's own, so that a store's lanes are
+   neighbours. Straight from the lanes a 16-byte store leaves every other 16 bytes of its lines to the next one: MI355X,
+   rmsfold of 4096 columns with xw, xn and xo at 1000 / 4096 tokens 37.5 / 142 us that way, 18.6 / 70 so; smfold of 12288 with
+   xo 50.4 / 212 against 32.9 / 148. kf_out: columns that t already holds */
+__device__ __forceinline__ void kf_put8(float* t, const float* v, int l){
+  *(float4*)(t + 8 * l) = make_float4(v[0], v[1], v[2], v[3]);
+  *(float4*)(t + 8 * l + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+__device__ __forceinline__ void kf_out(float* p, const float* t, int l, bool vec){
   if(vec){
-    *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
-    *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+#pragma unroll
+    for(int i = 0; i < 2; ++i) *(float4*)(p + 256 * i + 4 * l) = *(const float4*)(t + 256 * i + 4 * l);
   } else
 #pragma unroll
-    for(int i = 0; i < 8; ++i) p[i] = v[i];
+    for(int i = 0; i < 8; ++i) p[64 * i + l] = t[64 * i + l];
+}
+__device__ __forceinline__ void kf_st8(float* p, float* t, const float* v, int l, bool vec){
+  kt_wave_sync();                                                  /* t's earlier columns are read */
+  kf_put8(t, v, l);
+  kt_wave_sync();
+  kf_out(p, t, l, vec);
+  kt_wave_sync();
 }
 __device__ __forceinline__ void kf_stq(int8_t* p, const int* q, bool vec){
   if(vec){
@@ -248,14 +265,15 @@ __device__ __forceinline__ void kf_stq(int8_t* p, const int* q, bool vec){
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(512) k_fold_many(const KtFoldArgs a, int vec){
-  extern __shared__ __attribute__((aligned(16))) float kf_lds[];    /* [2][8][64][4] exchange, then (rmsfold) the row */
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE == 0 ? 6 : MODE == 2 ? 5 : 2))) k_fold_many(const KtFoldArgs a, int vec){
+  extern __shared__ __attribute__((aligned(16))) float kf_lds[];    /* [8][2][64][4] exchange (2 KB a wave), then the row */
   __shared__ double red[16];
   float4* ex = (float4*)kf_lds;
   float* rowb = kf_lds + 4096;
   const int j = threadIdx.x, n = blockIdx.y, l = j & 63, C = a.C, nw = a.HB >> 9;    /* nw waves an HB block: 1, 2, 8 */
   const int w = __builtin_amdgcn_readfirstlane(j >> 6);
   const bool vx = vec & KF_VX, vo = vec & KF_VO, vq = vec & KF_VQ;
+  float* tw = kf_lds + 512 * w;                                     /* this wave's part of the exchange */
   float s = 1.0f;
   if(MODE == 0){
     const float* x = a.x + (long long)n * a.ldx;
@@ -308,27 +326,30 @@ __global__ void __launch_bounds__(512) k_fold_many(const KtFoldArgs a, int vec){
     for(int c = 512 * w + 8 * l; c < C; c += 4096){
       float f[8];
       silu(c, f);
-      kf_st8(rowb + c, f, true);
+      kf_put8(rowb + c - 8 * l, f, l);
     }
     __syncthreads();
   }
   for(int c0 = whole ? 0 : blockIdx.x * 4096; c0 < (whole ? C : (int)blockIdx.x * 4096 + 1); c0 += 4096){
-    const int c = c0 + 512 * w + 8 * l;
+    const int cb = c0 + 512 * w, c = cb + 8 * l;                   /* the wave's columns (uniform), the lane's */
     const bool on = c0 + 512 * w < C;                              /* wave-uniform */
     float v[8];
 #pragma unroll
     for(int i = 0; i < 8; ++i) v[i] = 0.0f;
     if(on){
+      if(MODE == 0 && a.xw && a.nparts > 0){                       /* before the loads below: fewer registers at once */
+        kf_out(a.xw + (long long)n * a.ldxw + cb, rowb + cb, l, vo);
+        kt_wave_sync();
+      }
       float sg[8];
       kf_ld8(sg, a.sg + c, vx);
       if(MODE == 0){
         float f[8], wv[8];
         kf_ld8(f, rowb + c, true);
         kf_ld8(wv, a.w + c, vx);
-        if(a.xw && a.nparts > 0) kf_st8(a.xw + (long long)n * a.ldxw + c, f, vo);
 #pragma unroll
         for(int i = 0; i < 8; ++i) f[i] = (f[i] * s) * wv[i];
-        if(a.xn) kf_st8(a.xn + (long long)n * a.ldxn + c, f, vo);
+        if(a.xn) kf_st8(a.xn + (long long)n * a.ldxn + cb, tw, f, l, vo);
 #pragma unroll
         for(int i = 0; i < 8; ++i) v[i] = sg[i] * f[i];
       } else if(MODE == 1){
@@ -354,8 +375,8 @@ __global__ void __launch_bounds__(512) k_fold_many(const KtFoldArgs a, int vec){
 #undef KF_STAGE
     }
     if(nw > 1){                                                    /* uniform */
-      ex[w * 64 + l] = make_float4(v[0], v[1], v[2], v[3]);
-      ex[512 + w * 64 + l] = make_float4(v[4], v[5], v[6], v[7]);
+      ex[w * 128 + l] = make_float4(v[0], v[1], v[2], v[3]);
+      ex[w * 128 + 64 + l] = make_float4(v[4], v[5], v[6], v[7]);
       __syncthreads();
       if(on)
 #pragma unroll
@@ -364,7 +385,7 @@ __global__ void __launch_bounds__(512) k_fold_many(const KtFoldArgs a, int vec){
 #pragma unroll
           for(int t = 0; t < 8; ++t)
             if(t < 2 || nw > 2){
-              const float4 f = ex[512 * hf + ((w ^ t) & 7) * 64 + l];
+              const float4 f = ex[((w ^ t) & 7) * 128 + 64 * hf + l];
               A[t][0] = f.x; A[t][1] = f.y; A[t][2] = f.z; A[t][3] = f.w;
             }
 #pragma unroll
@@ -390,7 +411,6 @@ __global__ void __launch_bounds__(512) k_fold_many(const KtFoldArgs a, int vec){
         v[i] = v[i] * sc;
         m = i == 0 ? fabsf(v[0]) : fmaxf(m, fabsf(v[i]));
       }
-      if(a.xo) kf_st8(a.xo + (long long)n * a.ldxo + c, v, vo);
       m = fmaxf(m, kf_xorf<1>(m)); m = fmaxf(m, kf_xorf<2>(m)); m = fmaxf(m, kf_xorf<4>(m)); m = fmaxf(m, kf_xorf<8>(m));
       const float id = m != 0.0f ? 127.0f / m : 0.0f, xs = m / 127.0f;
       const long long n0 = a.hp ? 2 * (long long)n : n;
@@ -414,6 +434,7 @@ __global__ void __launch_bounds__(512) k_fold_many(const KtFoldArgs a, int vec){
         sum2 += kf_xor<1>(sum2); sum2 += kf_xor<2>(sum2); sum2 += kf_xor<4>(sum2); sum2 += kf_xor<8>(sum2);
         if((l & 15) == 0){ a.XS[(n0 + 1) * NG + g] = m / 32258.0f; a.XA[(n0 + 1) * NG + g] = sum2; }
       }
+      if(a.xo) kf_st8(a.xo + (long long)n * a.ldxo + cb, tw, v, l, vo);
     }
   }
 }
