@@ -452,7 +452,12 @@ template __global__ void k_fold_many<1>(const KtFoldArgs, int);
 template __global__ void k_fold_many<2>(const KtFoldArgs, int);
 
 #define KF_KEY(MODE, NM, NF) ((MODE) * 1024 + (NM) * 32 + (NF))
-#define KF_FEW 32                     /* up to this many tokens, one HB block a chunk */
+#define KF_FEW 32                     /* up to this many tokens, k_fold_q8 with one HB block a chunk */
+/* ... and rows of up to KF_NARROW columns at any number of tokens, where k_fold_many would leave 6 or 7 of a block's 8 waves
+   without columns of their own (MI355X, 64 / 4096 tokens, k_fold_many against k_fold_q8: rmsfold of 512 columns with one part
+   4.3 / 19.6 -> 3.6 / 15.0 us, of 1024 in HB 1024 4.8 / 26.5 -> 4.2 / 21.7, smfold 3.6 / 13.7 -> 3.1 / 10.9 and 4.1 / 23.7 -> 3.8 /
+   18.1). Not fold (512: 3.0 / 9.8 us on k_fold_q8, 2.9 / 5.5 on k_fold_many), nor smfold of two HB blocks (18.3 against 17.0) */
+#define KF_NARROW 1024
 
 /* host launcher (kt_api.hip validates the arguments) */
 static bool kf_overlap(const float* p, int ldp, const float* q, int ldq, int M, int C){
@@ -463,7 +468,6 @@ static bool kf_overlap(const float* p, int ldp, const float* q, int ldq, int M, 
 }
 
 hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
-  const int cw = a.HB;
   /* rmsfold over chunks of a row: every chunk's block reads the whole row (x and the parts, for the norm) while it
      writes its own chunk of xw / xn / xo. When one of those outputs overlaps x or the parts, one block takes the row
      (each thread writes only the columns it has read), so no block can overwrite what another has still to read. */
@@ -471,7 +475,8 @@ hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
   const bool alias = mode == 0 && (kf_overlap(a.xw, a.ldxw, a.x, a.ldx, M, a.C) || kf_overlap(a.xn, a.ldxn, a.x, a.ldx, M, a.C)
       || kf_overlap(a.xo, a.ldxo, a.x, a.ldx, M, a.C) || (np && (kf_overlap(a.xw, a.ldxw, a.r, a.ldr, M, np * a.C)
       || kf_overlap(a.xn, a.ldxn, a.r, a.ldr, M, np * a.C) || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, np * a.C))));
-  if(M > KF_FEW || alias){
+  const bool narrow = a.C <= KF_NARROW && (mode == 0 || (mode == 2 && a.C == a.HB));
+  if((M > KF_FEW || alias) && !narrow){
     auto al = [](const void* p, int ld, int b){ return (uintptr_t)p % b == 0 && (long long)ld * (b == 8 ? 1 : 4) % b == 0; };
     int vec = 0;
     if(al(a.x, a.ldx, 16) && (!a.r || al(a.r, a.ldr, 16)) && al(a.sg, 0, 16) && (!a.w || al(a.w, 0, 16))) vec |= KF_VX;
@@ -486,6 +491,7 @@ hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
     const dim3 grid(row ? 1 : (a.C + 4095) / 4096, M);
     return kt_go(mode == 0 ? k_fold_many<0> : mode == 1 ? k_fold_many<1> : k_fold_many<2>, grid, dim3(512), lds, s, a, vec);
   }
+  const int cw = narrow && (alias || (long long)M * (a.C / a.HB) > 512) ? a.C : a.HB;      /* past 2 blocks a CU, the row */
   const int nm = cw >> 9, nf = mode == 0 ? a.C >> 9 : nm;
   void (*k)(const KtFoldArgs) = nullptr;
   switch(KF_KEY(mode, nm, nf)){

@@ -1,5 +1,5 @@
-"""The input producers' many-token kernel (more than 32 tokens, or rmsfold with an output over its input) against the
-few-token one on the same rows: 8 columns a thread instead of one changes no pair of the transform and no order of the norm,
+"""The input producers' many-token kernel (more than 32 tokens, or rmsfold with an output over its input, of rows that are not
+narrow) against the few-token one on the same rows: 8 columns a thread instead of one changes no pair of the transform and no order of the norm,
 so every output has the same bits; odd strides and alignments take its scalar loads and stores."""
 import numpy as np
 import pytest
@@ -64,11 +64,35 @@ def test_many_equals_few(C, HB, hp, pad, shift):
             assert _same(t, torch.cat([f[k] for f in few])), (k, order)
 
 
+@pytest.mark.parametrize("C,HB,few", [(512, 512, "rmsfold smfold"), (1024, 1024, "rmsfold smfold"), (1024, 512, "rmsfold"), (1536, 512, ""),
+                                      (2048, 1024, "")])
+def test_narrow_rows_route(C, HB, few):
+    """more than 32 tokens of narrow rows stay with the few-token kernel (no dynamic LDS): the other one's waves would idle"""
+    from kindi_amd import linear as lin
+    M = 40
+    x, sg = torch.randn((M, C), device="cuda"), torch.ones(C, device="cuda")
+    xw, act = torch.empty_like(x), _act(lin, M, C, False, 0)
+    calls = {"rmsfold": lambda: lin.rmsfold(x, sg, sg, HB, r=x, nparts=1, xw=xw, out=act),
+             "fold": lambda: lin.fold(x, sg, HB, out=act), "smfold": lambda: lin.smfold(x, x, sg, HB, out=act)}
+    for name, fn in calls.items():
+        plan = lin.Plan(fn, 2)
+        assert plan.n == 1 and (plan.recs[0].shmem == 0) == (name in few.split()), (name, plan.recs[0].shmem)
+
+
 def test_outputs_over_inputs():
     """rmsfold's outputs over x (any token count), smfold's xo over a in the grouped-head order (one block a row)"""
     from kindi_amd import linear as lin
     M, C = 40, 6144
     r = rng(9)
+    for n, hb in ((512, 512), (1024, 512), (1024, 1024)):                # narrow rows: the few-token kernel, a block a row
+        x, b = (dev(r.standard_normal((M, n)).astype(np.float32)) for _ in range(2))
+        sg = dev(np.where(r.random(n) < 0.5, -1, 1).astype(np.float32))
+        for m in (1, M):
+            out = torch.empty((m, n), device="cuda")
+            a0 = lin.rmsfold(x[:m], sg, sg, hb, r=b[:m], nparts=1, xw=out)
+            y = x[:m].clone()
+            a1 = lin.rmsfold(y, sg, sg, hb, r=b[:m], nparts=1, xw=y)
+            assert _same(y, out) and _same(a0.XQ, a1.XQ) and _same(a0.XS, a1.XS)
     x, b = (dev(r.standard_normal((M, C)).astype(np.float32)) for _ in range(2))
     w, sg = torch.ones(C, device="cuda"), dev(np.where(r.random(C) < 0.5, -1, 1).astype(np.float32))
     for m in (1, M):
