@@ -258,7 +258,8 @@ int kt_moe_decode_noalloc(const void* const* Wup, const void* const* Wdown, int 
    fold = the unnormalised Walsh-Hadamard transform of each HB-column block times 1/sqrt(HB), HB in {512, 1024,
    4096}. C % HB == 0; rmsfold takes C <= 8192 (one block holds the row for the norm), fold / smfold any width up to
    2^20 (chunks of whole HB blocks). M <= 65535. xw (x + parts, only with nparts > 0), xn and xo are nullable;
-   xw, xn and xo may be x itself (with its row stride); they may not overlap x or the parts otherwise.
+   xw, xn and xo may be x itself (with its row stride; smfold's xo: a or b); they may not overlap x or the parts otherwise.
+   smfold in place with rep > 1 and nk > 1 holds a row's inputs in LDS: up to 36352 columns, hipErrorInvalidValue beyond.
    HB | KT_HP: the reference's two-row form (hp, ff_q8 tcf.cu:150-205): XQ / XS / XA with 2M rows, row 2n the int8
    row above, row 2n + 1 the residual r = fma(-q, amax / 127, xo) at the fixed scale amax / 32258:
    q2 = clamp(rne(r (32258 / amax)), -127, 127), XS = amax / 32258, XA = sum q2 (0 when amax = 0). */

@@ -458,6 +458,7 @@ template __global__ void k_fold_many<2>(const KtFoldArgs, int);
    4.3 / 19.6 -> 3.6 / 15.0 us, of 1024 in HB 1024 4.8 / 26.5 -> 4.2 / 21.7, smfold 3.6 / 13.7 -> 3.1 / 10.9 and 4.1 / 23.7 -> 3.8 /
    18.1). Not fold (512: 3.0 / 9.8 us on k_fold_q8, 2.9 / 5.5 on k_fold_many), nor smfold of two HB blocks (18.3 against 17.0) */
 #define KF_NARROW 1024
+#define KF_ROW_MAX 36352              /* columns of a row in LDS beside the exchange (160 KB a CU) */
 
 /* host launcher (kt_api.hip validates the arguments) */
 static bool kf_overlap(const float* p, int ldp, const float* q, int ldq, int M, int C){
@@ -475,18 +476,20 @@ hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
   const bool alias = mode == 0 && (kf_overlap(a.xw, a.ldxw, a.x, a.ldx, M, a.C) || kf_overlap(a.xn, a.ldxn, a.x, a.ldx, M, a.C)
       || kf_overlap(a.xo, a.ldxo, a.x, a.ldx, M, a.C) || (np && (kf_overlap(a.xw, a.ldxw, a.r, a.ldr, M, np * a.C)
       || kf_overlap(a.xn, a.ldxn, a.r, a.ldr, M, np * a.C) || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, np * a.C))));
+  /* smfold's grouped-head order reads other chunks' columns (with one key group, nk 1, it is the plain order): where xo lies
+     over an input, a block takes the row, its inputs in LDS before an output is written, at any number of tokens */
+  const bool turned = mode == 2 && a.rep > 1 && a.nk > 1 && (kf_overlap(a.xo, a.ldxo, a.x, a.ldx, M, a.C)
+                      || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, a.C));
+  if(turned && a.C > KF_ROW_MAX) return hipErrorInvalidValue;
   const bool narrow = a.C <= KF_NARROW && (mode == 0 || (mode == 2 && a.C == a.HB));
-  if((M > KF_FEW || alias) && !narrow){
+  if((M > KF_FEW || alias || turned) && !narrow){
     auto al = [](const void* p, int ld, int b){ return (uintptr_t)p % b == 0 && (long long)ld * (b == 8 ? 1 : 4) % b == 0; };
     int vec = 0;
     if(al(a.x, a.ldx, 16) && (!a.r || al(a.r, a.ldr, 16)) && al(a.sg, 0, 16) && (!a.w || al(a.w, 0, 16))) vec |= KF_VX;
     if((!a.xw || al(a.xw, a.ldxw, 16)) && (!a.xn || al(a.xn, a.ldxn, 16)) && (!a.xo || al(a.xo, a.ldxo, 16))) vec |= KF_VO;
     if(al(a.Q, a.ldq, 8)) vec |= KF_VQ;
-    /* the grouped-head order reads other chunks' columns: where xo lies over an input, a block takes the row (up to 8192
-       columns, as the norm's kernel) */
-    if(mode == 2 && a.rep > 1 && a.C <= 8192 && (kf_overlap(a.xo, a.ldxo, a.x, a.ldx, M, a.C)
-       || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, a.C))) vec |= KF_ROW;
-    const bool row = mode == 0 || (vec & KF_ROW);
+    if(turned) vec |= KF_ROW;
+    const bool row = mode == 0 || turned;
     const size_t lds = 16384 + (row ? (size_t)a.C * 4 : 0);
     const dim3 grid(row ? 1 : (a.C + 4095) / 4096, M);
     return kt_go(mode == 0 ? k_fold_many<0> : mode == 1 ? k_fold_many<1> : k_fold_many<2>, grid, dim3(512), lds, s, a, vec);

@@ -80,7 +80,7 @@ def test_narrow_rows_route(C, HB, few):
 
 
 def test_outputs_over_inputs():
-    """rmsfold's outputs over x (any token count), smfold's xo over a in the grouped-head order (one block a row)"""
+    """rmsfold's outputs over x (any token count), narrow rows among them"""
     from kindi_amd import linear as lin
     M, C = 40, 6144
     r = rng(9)
@@ -101,8 +101,33 @@ def test_outputs_over_inputs():
         y = x[:m].clone()
         a1 = lin.rmsfold(y, w, sg, 1024, r=b[:m], nparts=1, xo=y)
         assert _same(y, out[2]) and _same(a0.XQ, a1.XQ) and _same(a0.XS, a1.XS)
-    want = torch.empty_like(x)
-    a0 = lin.smfold(x, b, sg, 1024, perm=(128, 24, 2), xo=want)
-    y = x.clone()
-    a1 = lin.smfold(y, b, sg, 1024, perm=(128, 24, 2), xo=y)
-    assert _same(y, want) and _same(a0.XQ, a1.XQ)
+
+
+# one token to more than the few-token kernel's 32, rows of one chunk and of several, up to the widest that LDS holds
+@pytest.mark.parametrize("M,C,HB,perm", [(1, 6144, 1024, (128, 24, 2)), (32, 6144, 1024, (128, 24, 2)), (40, 6144, 1024, (128, 24, 2)),
+                                         (1, 12288, 4096, (128, 16, 6)), (40, 12288, 4096, (128, 16, 6)), (3, 1024, 1024, (128, 2, 4)),
+                                         (3, 1024, 512, (128, 2, 4)), (2, 36352, 512, (256, 2, 71)), (2, 35840, 1024, (256, 20, 7)), (2, 32768, 4096, (128, 128, 2))])
+@pytest.mark.parametrize("over", ["a", "b"])
+def test_smfold_in_place_grouped_heads(M, C, HB, perm, over):
+    """smfold's xo over one of its inputs in the grouped-head order, where a chunk reads other chunks' columns: the outputs
+    of the call with an xo of its own"""
+    from kindi_amd import linear as lin
+    say("smfold in place", M, C, HB, perm, over)
+    r = rng(C + M)
+    a, b = (dev(r.standard_normal((M, C)).astype(np.float32)) for _ in range(2))
+    sg = dev(np.where(r.random(C) < 0.5, -1, 1).astype(np.float32))
+    want = torch.empty_like(a)
+    a0 = lin.smfold(a, b, sg, HB, perm=perm, xo=want)
+    y = (a if over == "a" else b).clone()
+    a1 = lin.smfold(y if over == "a" else a, y if over == "b" else b, sg, HB, perm=perm, xo=y)
+    assert _same(y, want) and all(_same(u, v) for u, v in zip((a0.XQ, a0.XS, a0.XA), (a1.XQ, a1.XS, a1.XA)))
+
+
+def test_smfold_in_place_refused_past_lds():
+    from kindi_amd import gpudrv, linear as lin
+    C, sg = 36864, torch.ones(36864, device="cuda")
+    a, b = torch.randn((1, C), device="cuda"), torch.randn((1, C), device="cuda")
+    with pytest.raises(gpudrv.KernelError):
+        lin.smfold(a, b, sg, 512, perm=(128, 144, 2), xo=a)
+    lin.smfold(a, b, sg, 512, perm=(128, 144, 2), xo=torch.empty_like(a))       # not in place, and the plain order: taken
+    lin.smfold(a, b, sg, 512, perm=(18432, 1, 2), xo=a)
