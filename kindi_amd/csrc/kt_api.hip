@@ -35,8 +35,8 @@ __global__ void k_q8_gemm(const KtGemvArgs, const KtGroupedArgs, const int8_t*, 
 template <int SRC> __global__ void k_tern_pack(const uint8_t*, const uint16_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_q8_pack(const uint8_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_tern_pack_ptq1(const uint8_t*, int, int, int, int, uint32_t*, uint16_t*);
-template <bool HP> __global__ void k_quant_tern(const float*, int, int, int, int8_t*, int, float*, int*);
-template <int NR> __global__ void k_quant_row(const float*, int, int, int8_t*, int, float*, int*);
+template <bool HP, bool SH> __global__ void k_quant_tern(const float*, int, int, int, int8_t*, int, float*, int*);
+template <int NR, int W> __global__ void k_quant_row(const float*, int, int, int8_t*, int, float*, int*);
 extern "C" __global__ void k_quant_q8(const float*, int, int, int, int8_t*, int, float*, int);
 extern "C" __global__ void k_tern_sum(const float*, float*, int, int, int);
 template <int NW, bool RS, bool DBG>
@@ -529,9 +529,10 @@ int kt_quant_q8(const float* X, int ldx, int M, int C, int per_row, int8_t* XQ, 
       int8_t* q = XQ + (long long)m0 * ldq;
       float* xs = XS + (long long)m0 * NG;
       int* xa = (int*)XA + (long long)m0 * NG;
-#define KT_QR(NR) KT_LAUNCH((k_quant_row<NR>), grid, dim3(512), 0, s, x, ldx, C, q, ldq, xs, xa)
-      if(nr <= 4) KT_QR(4); else if(nr <= 8) KT_QR(8); else if(nr <= 16) KT_QR(16); else if(nr <= 32) KT_QR(32);
-      else KT_QR(0);
+#define KT_QR(NR, W) KT_LAUNCH((k_quant_row<NR, W>), grid, dim3(64 * W), 0, s, x, ldx, C, q, ldq, xs, xa)
+      if(NG <= 1) KT_QR(1, 1); else if(NG <= 2) KT_QR(1, 2); else if(NG <= 4) KT_QR(1, 4);
+      else if(nr <= 4) KT_QR(4, 8); else if(nr <= 8) KT_QR(8, 8); else if(nr <= 16) KT_QR(16, 8); else if(nr <= 32) KT_QR(32, 8);
+      else KT_QR(0, 8);
 #undef KT_QR
     }
     return 0;
@@ -539,8 +540,11 @@ int kt_quant_q8(const float* X, int ldx, int M, int C, int per_row, int8_t* XQ, 
   /* chunks of a row: one group a wave while the rows are few, down to one block a row from 4096 rows (16 blocks of 4
      waves a CU) */
   const int most = (NG + 3) / 4, want = 4096 / M > 1 ? 4096 / M : 1, nch = want < most ? want : most;
-  if(per_row == 2) KT_LAUNCH((k_quant_tern<true>), dim3(M * nch), dim3(256), 0, s, X, ldx, C, nch, XQ, ldq, XS, (int*)XA);
-  else KT_LAUNCH((k_quant_tern<false>), dim3(M * nch), dim3(256), 0, s, X, ldx, C, nch, XQ, ldq, XS, (int*)XA);
+  const dim3 block(64 * (NG < 4 ? NG : 4));
+#define KT_QT(HP, SH) KT_LAUNCH((k_quant_tern<HP, SH>), dim3(M * nch), block, 0, s, X, ldx, C, nch, XQ, ldq, XS, (int*)XA)
+  if(per_row == 2){ if(nch == 1 && NG >= 16) KT_QT(true, true); else KT_QT(true, false); }
+  else KT_QT(false, false);
+#undef KT_QT
   return 0;
 }
 

@@ -152,14 +152,21 @@ extern "C" __global__ void k_q8_pack(const uint8_t* __restrict__ rows, int R, in
 
 /* ------------------------------------------------------------------ activations */
 /* one 128-column group of a row by one wave: lane l holds columns 2 l, 2 l + 1 (v) and the scale's amax; HP: the
-   residual's row too (per_row 2 below). n0: the group's first output row */
-template <bool HP>
+   residual's row too (per_row 2 below). n0: the group's first output row. SH: the sums over the wave through the LDS
+   crossbar instead of the VALU, which leaves the VALU to the other waves but takes longer */
+template <bool SH> __device__ __forceinline__ int kt_quant_sum(int v){
+  if(!SH) return kf_wave_sum(v);
+#pragma unroll
+  for(int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+template <bool HP, bool SH = false>
 __device__ __forceinline__ void kt_quant_group(float2 v, float amax, long long n0, int g, int NG, int lane,
                                                int8_t* __restrict__ Q, int ldq, float* __restrict__ XS,
                                                int* __restrict__ XA){
   const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
   const int q0 = __float2int_rn(v.x * id), q1 = __float2int_rn(v.y * id);
-  const int s = kf_wave_sum(q0 + q1);
+  const int s = kt_quant_sum<SH>(q0 + q1);
   *(uint16_t*)(Q + n0 * ldq + g * 128 + 2 * lane) = (uint16_t)((q0 & 255) | ((q1 & 255) << 8));
   if(lane == 0){
     XS[n0 * NG + g] = amax / 127.0f;
@@ -169,7 +176,7 @@ __device__ __forceinline__ void kt_quant_group(float2 v, float amax, long long n
     const float sc = amax / 127.0f, a2 = amax / 254.0f, id2 = a2 != 0.0f ? 127.0f / a2 : 0.0f;
     const float r0 = fmaf(-(float)q0, sc, v.x), r1 = fmaf(-(float)q1, sc, v.y);
     const int p0 = max(-127, min(127, __float2int_rn(r0 * id2))), p1 = max(-127, min(127, __float2int_rn(r1 * id2)));
-    const int s2 = kf_wave_sum(p0 + p1);
+    const int s2 = kt_quant_sum<SH>(p0 + p1);
     *(uint16_t*)(Q + (n0 + 1) * ldq + g * 128 + 2 * lane) = (uint16_t)((p0 & 255) | ((p1 & 255) << 8));
     if(lane == 0){
       XS[(n0 + 1) * NG + g] = a2 / 127.0f;
@@ -182,12 +189,15 @@ __device__ __forceinline__ void kt_quant_group(float2 v, float amax, long long n
    groups 4 (b % nch) + w, + 4 nch, ..., KT_QB of them loaded together. nch: as many chunks as give the GPU blocks enough
    (kt_quant_q8), so that a row's groups are not quantized one after the other by four waves when the rows are few:
    MI355X, 4 tokens of 12288 columns in the two-row form 10.3 -> 4.2 us, one token of 6144 columns 3.9 -> 2.6 us, 61
-   tokens of 5120 columns 9.4 -> 3.4 us (dependent launches).
+   tokens of 5120 columns 9.4 -> 3.4 us (dependent launches). KT_QB 2 and only real groups loaded: with 4, past the row's end the
+   first one again, 5000 rows of 512 columns took 7.1 us (5.7 so, 6.5 one group at a time), 1000 of 2048 6.1 (5.0, 5.3).
+   Waves: 4, or the row's groups where those are fewer. SH (the two-row form, a block a row, 16 groups and more: there the
+   VALU bounds it): 5000 rows of 6144 columns 61.8 -> 55.4 us; at fewer rows it adds 0.3 us to each launch.
    HP (per_row 2, k_tc_q8 with hp, tc.cu:195-209): two rows a token, 2n the group's int8 row, 2n + 1 its residual
    r = v - q (amax / 127) (one fma, as the reference's compiler contracts it) quantized with the fixed amax
    a2 = amax / 254: q2 = clamp(rne(r (127 / a2)), -127, 127), XS = a2 / 127, XA = sum q2 (tcq128 tc.cu:160-194). */
-#define KT_QB 4
-template <bool HP>
+#define KT_QB 2
+template <bool HP, bool SH>
 __global__ void __launch_bounds__(256) k_quant_tern(const float* __restrict__ X, int ldx, int C, int nch,
                                                     int8_t* __restrict__ Q, int ldq, float* __restrict__ XS,
                                                     int* __restrict__ XA){
@@ -200,40 +210,43 @@ __global__ void __launch_bounds__(256) k_quant_tern(const float* __restrict__ X,
 #pragma unroll
     for(int i = 0; i < KT_QB; ++i){
       const int g = g0 + 4 * nch * i;
-      v[i] = *(const float2*)(x + (g < NG ? g : g0) * 128 + 2 * lane);
+      if(g < NG) v[i] = *(const float2*)(x + g * 128 + 2 * lane);
     }
 #pragma unroll
     for(int i = 0; i < KT_QB; ++i){
       const int g = g0 + 4 * nch * i;
-      if(g < NG) kt_quant_group<HP>(v[i], kf_wave_max(fmaxf(fabsf(v[i].x), fabsf(v[i].y))), n0, g, NG, lane, Q, ldq, XS, XA);
+      if(g < NG) kt_quant_group<HP, SH>(v[i], kf_wave_max(fmaxf(fabsf(v[i].x), fabsf(v[i].y))), n0, g, NG, lane, Q, ldq, XS, XA);
     }
   }
 }
-template __global__ void k_quant_tern<false>(const float*, int, int, int, int8_t*, int, float*, int*);
-template __global__ void k_quant_tern<true>(const float*, int, int, int, int8_t*, int, float*, int*);
+template __global__ void k_quant_tern<false, false>(const float*, int, int, int, int8_t*, int, float*, int*);
+template __global__ void k_quant_tern<true, false>(const float*, int, int, int, int8_t*, int, float*, int*);
+template __global__ void k_quant_tern<true, true>(const float*, int, int, int, int8_t*, int, float*, int*);
 
-/* One scale a token row (per_row 1): grid (M), block 512: wave w holds groups w, w + 8, ... in registers (NR of them,
-   all loaded before the row's amax is known), so the row is read once: MI355X, 2048 rows of 12288 columns 25 us
-   (read twice: 37.7), of 4096 columns 10 us (16.5). Rows of more than 8 NR groups read it again (NR = 0). */
-template <int NR>
-__global__ void __launch_bounds__(512) k_quant_row(const float* __restrict__ X, int ldx, int C, int8_t* __restrict__ Q,
+/* One scale a token row (per_row 1): grid (M), a block of W waves: wave w holds groups w, w + W, ... in registers (NR of
+   them, all loaded before the row's amax is known), so the row is read once: MI355X, 2048 rows of 12288 columns 25 us
+   (read twice: 37.7), of 4096 columns 10 us (16.5). Rows of more than 256 groups read it again (NR = 0). W = 8, for rows of up
+   to 4 groups 1, 2 or 4: 16384 rows of 128 columns 19.7 us in blocks of 8 waves, 11.4 of 4, 6.1 of one; of 512 22.2 -> 13.3. W is a
+   constant: counted at run time it cost every width 0.2 us. */
+template <int NR, int W>
+__global__ void __launch_bounds__(64 * W) k_quant_row(const float* __restrict__ X, int ldx, int C, int8_t* __restrict__ Q,
                                                    int ldq, float* __restrict__ XS, int* __restrict__ XA){
   const int n = blockIdx.x, lane = threadIdx.x & 63, NG = C >> 7;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float* x = X + (long long)n * ldx;
-  __shared__ float red[8];
+  __shared__ float red[W];
   float2 v[NR > 0 ? NR : 1];
   float a = 0.0f;
   if(NR > 0){
 #pragma unroll
     for(int i = 0; i < NR; ++i){
-      const int g = w + 8 * i;
+      const int g = w + W * i;
       v[i] = g < NG ? *(const float2*)(x + g * 128 + 2 * lane) : make_float2(0.0f, 0.0f);
     }
 #pragma unroll
     for(int i = 0; i < NR; ++i) a = fmaxf(a, fmaxf(fabsf(v[i].x), fabsf(v[i].y)));
   } else
-    for(int g = w; g < NG; g += 8){
+    for(int g = w; g < NG; g += W){
       const float2 u = *(const float2*)(x + g * 128 + 2 * lane);
       a = fmaxf(a, fmaxf(fabsf(u.x), fabsf(u.y)));
     }
@@ -242,17 +255,17 @@ __global__ void __launch_bounds__(512) k_quant_row(const float* __restrict__ X, 
   __syncthreads();
   float amax = red[0];
 #pragma unroll
-  for(int i = 1; i < 8; ++i) amax = fmaxf(amax, red[i]);
+  for(int i = 1; i < W; ++i) amax = fmaxf(amax, red[i]);
   if(NR > 0){
 #pragma unroll
     for(int i = 0; i < NR; ++i)
-      if(w + 8 * i < NG) kt_quant_group<false>(v[i], amax, n, w + 8 * i, NG, lane, Q, ldq, XS, XA);
+      if(w + W * i < NG) kt_quant_group<false>(v[i], amax, n, w + W * i, NG, lane, Q, ldq, XS, XA);
   } else
-    for(int g = w; g < NG; g += 8)
+    for(int g = w; g < NG; g += W)
       kt_quant_group<false>(*(const float2*)(x + g * 128 + 2 * lane), amax, n, g, NG, lane, Q, ldq, XS, XA);
 }
-#define KT_QR(NR) template __global__ void k_quant_row<NR>(const float*, int, int, int8_t*, int, float*, int*);
-KT_QR(0) KT_QR(4) KT_QR(8) KT_QR(16) KT_QR(32)
+#define KT_QR(NR, W) template __global__ void k_quant_row<NR, W>(const float*, int, int, int8_t*, int, float*, int*);
+KT_QR(1, 1) KT_QR(1, 2) KT_QR(1, 4) KT_QR(0, 8) KT_QR(4, 8) KT_QR(8, 8) KT_QR(16, 8) KT_QR(32, 8)
 #undef KT_QR
 
 /* grid (ceil(C/32 / 8), M), block 256: a group of 32 lanes quantizes one 32-column block (llama.cpp's CPU q8_0

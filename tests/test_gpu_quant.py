@@ -40,3 +40,16 @@ def test_group_chunks(NG, M, mode):
     X[0, :128] = 0.0
     X[-1] *= 1e-30
     _same(X, mode, 6)
+
+
+# rows of fewer groups than a block has waves otherwise (blocks of 1, 2 and 4 waves per row, of NG per group), and the two-row form
+# around the line at which its sums go over the LDS crossbar (16 groups, 4096 rows)
+@pytest.mark.parametrize("NG,M,mode", [(1, 3, 1), (2, 5, 1), (3, 5, 1), (4, 6, 1), (5, 5, 1), (2, 4100, 1), (1, 4100, 0), (2, 9, 0), (3, 4096, 2),
+                                       (15, 4096, 2), (16, 4095, 2), (16, 4096, 2), (17, 4099, 2)])
+def test_narrow_rows_and_two_row_line(NG, M, mode):
+    say("quant narrow", NG, M, mode)
+    X = rng(NG * M).normal(0, 1, (M, NG * 128)).astype(np.float32)
+    X[0, -128:] = 0.0
+    X[1, :128] *= 1e4
+    X[2] *= 1e-30
+    _same(X, mode, 2)
