@@ -53,7 +53,7 @@ size_t kt_gemm8_lds();
 __global__ void k_moe_topk(const float*, int, int, const KtRouter, int*, float*);
 extern "C" __global__ void k_moe_sort(const int*, int, int, int*, int*, int*, int*, int*, int*, int);
 extern "C" __global__ void k_moe_combine(const float*, const float*, const int*, const float*, int, int, float*, int);
-__global__ void k_moe_route(const float*, int, int, int, const KtRouter, int*, float*, int*, int*, int*, int*, int*,
+template <bool X> __global__ void k_moe_route(const float*, int, int, int, const KtRouter, int*, float*, int*, int*, int*, int*, int*,
                             int*, const float*, int, int, int8_t*, int, float*, int);
 __global__ void k_moe1_up(const float*, int, int, const KtRouter, const uint8_t* const*, const uint8_t* const*, int,
                           int, const float*, float*, int*, float*, const uint8_t**, int);
@@ -332,7 +332,7 @@ static int kt_moe_decode_run(const void* const* Wup, const void* const* Wdown, i
     return 0;
   }
   /* 1: router, top-k, lists */
-  KT_LAUNCH(k_moe_route, dim3(1), dim3(KT_RT_BLOCK), 0, s, logits, M, E, k, rt, ids, gw, cnt, off, xrow, where, act, nact,
+  KT_LAUNCH(k_moe_route<false>, dim3(1), dim3(KT_RT_BLOCK), 0, s, logits, M, E, k, rt, ids, gw, cnt, off, xrow, where, act, nact,
                      (const float*)nullptr, 0, 0, (int8_t*)nullptr, 0, (float*)nullptr, 0);
   const int n = M * k;
   /* 2: up = W_e x[xrow[p]] per entry, x quantized in the staging */
@@ -790,8 +790,8 @@ int kt_moe_route_r(const float* logits, int M, int E, int k, int score, const fl
   if(!logits || !ids || !gw || !cnt || !off || !xrow || !where || !act || !nact || M < 0 || E <= 0 || E > 1024 ||
      k <= 0 || k > 16 || k > E || M > 64 || (long long)M * k > 64) return KT_INVALID;
   if(x && (H <= 0 || H % 32 || ldx < H || !Q || ldq < H || !D || ldd < H / 32)) return KT_INVALID;
-  KT_LAUNCH(k_moe_route, dim3(1), dim3(KT_RT_BLOCK), 0, kt_stream(stream), logits, M, E, k, rt, ids, gw, cnt, off, xrow,
-            where, act, nact, x, ldx, H, Q, ldq, D, ldd);
+  KT_LAUNCH(x ? k_moe_route<true> : k_moe_route<false>, dim3(1), dim3(KT_RT_BLOCK), 0, kt_stream(stream), logits, M, E, k, rt,
+            ids, gw, cnt, off, xrow, where, act, nact, x, ldx, H, Q, ldq, D, ldd);
   return 0;
 }
 

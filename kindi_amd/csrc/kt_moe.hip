@@ -122,6 +122,7 @@ extern "C" __global__ void __launch_bounds__(1024) k_moe_sort(const int* __restr
    as kt_moe_sort), their count; lane l owns experts l per .. + per - 1 (per = ceil(E / 64)), offsets and the active list
    by prefix sums over lanes. The same outputs as k_moe_topk + k_moe_sort. */
 #define KT_RT_WAVES 8
+template <bool X>   /* x given */
 __global__ void __launch_bounds__(64 * KT_RT_WAVES) k_moe_route(const float* __restrict__ logits, int M, int E, int k,
     const KtRouter rt, int* __restrict__ ids, float* __restrict__ gw, int* __restrict__ cnt, int* __restrict__ off,
     int* __restrict__ xrow, int* __restrict__ where, int* __restrict__ act, int* __restrict__ nact,
@@ -134,37 +135,57 @@ __global__ void __launch_bounds__(64 * KT_RT_WAVES) k_moe_route(const float* __r
     if(lane < k) pick[t * k + lane] = mine;
   }
   for(int e = threadIdx.x; e < E; e += blockDim.x) c[e] = 0;
-  __syncthreads();
-  if(w > 0){
-    /* the other waves: the tokens' int8 rows, k_quant_q8's numbers (act 0): a 32-lane half per 32-column block */
-    if(!x) return;
-    /* blocks h, h + nh, ... of every token, KT_RQ at a time: their loads issued together (clamped to a real block),
-       then the reductions and stores, so a half-wave waits for memory once per KT_RQ blocks, not once per block */
-    const int h = (threadIdx.x - 64) >> 5, nh = 2 * (W - 1), l = threadIdx.x & 31, nb = H / 32;
-    constexpr int KT_RQ = 8;
-    for(int t = 0; t < M; ++t)
-      for(int b0 = h; b0 < nb; b0 += nh * KT_RQ){
-        float v[KT_RQ];
+  /* the tokens' int8 rows, k_quant_q8's numbers (act 0): 16 blocks of 32 columns of one token at a time (512 columns), a
+     32-lane half a block, so that a wave waits for memory once for 512 columns; by waves 1 .. while wave 0 builds the lists, the
+     first ones' loads before the barrier. early: one or two tokens of many experts, where the top-k is the longer part (7 us
+     at 512): the waves without a token, during the others' top-k. MI355X, 128 experts, 6 picks, x of 1024 / 2688 / 7168 columns:
+     1 token 4.7 / 5.2 / 7.1 us, 7 tokens 7.9 / 14.9 / 30.9, 10 tokens 11.1 / 20.3 / 43.5 (token after token
+     by all 7 waves, 112 blocks' work each time: 4.8 / 5.3 / 7.6, 12.6 / 16.0 / 31.5, 17.9 / 22.5 / 44.7; by three waves beside one that
+     does every token's top-k: 5.6 / 5.7 / 8.6, 21.4 / 21.6 / 50.0, 29.2 / 29.5 / 70.7) */
+  if(X){
+    const int nb = H >> 5, nc = (nb + 15) >> 4, nq = M * nc, l = lane & 31, h = lane >> 5;
+    const bool early = 4 * M <= W && E > 256;                      /* uniform */
+    const int step = early ? W - M : W - 1;
+    int i = early ? w - M : w - 1;
+    const bool on = i >= 0 && i < nq;                              /* wave-uniform */
+    float v[8];
+    int qt = 0, qc = 0;                                            /* uniform: the token and the 512 columns v is of */
+    auto ld = [&]{
+      const float* xt = x + (long long)qt * ldx + qc * 512 + lane;
 #pragma unroll
-        for(int q = 0; q < KT_RQ; ++q){
-          const int b = b0 + nh * q;
-          v[q] = x[(long long)t * ldx + (b < nb ? b : b0) * 32 + l];
-        }
+      for(int q = 0; q < 8; ++q) v[q] = 16 * qc + 2 * q + h < nb ? xt[64 * q] : 0.0f;
+    };
+    if(on){
+      qt = i / nc;
+      qc = i - qt * nc;
+      ld();
+    }
+    if(!early) __syncthreads();
+    if(on)
+      for(; i < nq; i += step){
+        float u[8];
 #pragma unroll
-        for(int q = 0; q < KT_RQ; ++q){
-          const int b = b0 + nh * q;
-          float a = fabsf(v[q]);
+        for(int q = 0; q < 8; ++q) u[q] = v[q];
+        const int left = nb - 16 * qc - h;
+        int8_t* Qt = Q + (long long)qt * ldq + qc * 512 + lane;
+        float* Dt = D + (long long)qt * ldd + qc * 16 + h;
+        for(qc += step; qc >= nc; qc -= nc) ++qt;
+        if(i + step < nq) ld();
+#pragma unroll
+        for(int q = 0; q < 8; ++q){
+          float a = fabsf(u[q]);
           a = fmaxf(a, kf_xorf<1>(a)); a = fmaxf(a, kf_xorf<2>(a)); a = fmaxf(a, kf_xorf<4>(a));
           a = fmaxf(a, kf_xorf<8>(a)); a = fmaxf(a, kf_xorf<16>(a));
           const float id = a != 0.0f ? 127.0f / a : 0.0f;
-          if(b < nb){
-            Q[(long long)t * ldq + b * 32 + l] = (int8_t)__float2int_rn(v[q] * id);
-            if(l == 0) D[(long long)t * ldd + b] = __half2float(__float2half_rn(a / 127.0f));
+          if(2 * q < left){
+            Qt[64 * q] = (int8_t)__float2int_rn(u[q] * id);
+            if(l == 0) Dt[2 * q] = __half2float(__float2half_rn(a / 127.0f));
           }
         }
       }
-    return;
-  }
+    if(early) __syncthreads();
+  } else __syncthreads();
+  if(w > 0) return;
   const bool valid = lane < n;
   const int ep = valid ? pick[lane] : 0;
   unsigned long long eq = __ballot(valid);
@@ -211,6 +232,10 @@ __global__ void __launch_bounds__(64 * KT_RT_WAVES) k_moe_route(const float* __r
     where[lane] = pos;
   }
 }
+
+#define KT_RT(X) template __global__ void k_moe_route<X>(const float*, int, int, int, const KtRouter, int*, float*, int*, int*, \
+    int*, int*, int*, int*, const float*, int, int, int8_t*, int, float*, int);
+KT_RT(false) KT_RT(true)
 
 extern "C" __global__ void __launch_bounds__(256) k_moe_combine(const float* __restrict__ yd, const float* __restrict__ ysh,
     const int* __restrict__ where, const float* __restrict__ gw, int k, int cols, float* __restrict__ x, int ldx){

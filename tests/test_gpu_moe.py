@@ -442,3 +442,32 @@ def test_moe_decode_row_at_allocation_end(kt):
     want, _ = layer.forward(dev(x), dev(lg))
     layer.decode(xe, le)
     assert np.array_equal(host(xe).view(np.uint32), host(want).view(np.uint32))
+
+
+# x of one block, of blocks that do not fill a wave's 16, and of several such; more tokens than waves, and few tokens of many
+# experts (their int8 rows are made during the top-k); rows of a wider x, and outputs whose surroundings stay as they are
+@pytest.mark.parametrize("H", [32, 96, 512, 544, 1056, 7200])
+@pytest.mark.parametrize("M,E,k", [(1, 8, 2), (3, 128, 6), (8, 64, 8), (9, 60, 4), (64, 128, 1), (1, 512, 8), (2, 300, 3), (3, 1024, 16)])
+def test_route_quantizes_x(kt, M, E, k, H):
+    lib, moe = kt
+    say("route x", M, E, k, H)
+    from kindi_amd.linear import ptr, stream
+    lg = dev(rng(M + E).normal(0, 1, (M, E)).astype(np.float32))
+    wide = dev(rng(H + M).normal(0, 1, (M, H + 36)).astype(np.float32))
+    wide[0, :32] = 0.0
+    x = wide[:, :H]
+    iz = [torch.empty(n, dtype=torch.int32, device="cuda") for n in (M * k, E, E, M * k, M * k, E, 1)]
+    gw = torch.empty(M * k, device="cuda")
+    Q = torch.full((M + 1, H + 48), 77, dtype=torch.int8, device="cuda")
+    D = torch.full((M + 1, H // 32 + 3), -7.0, device="cuda")
+    assert lib.kt_moe_route_r(ptr(lg), M, E, k, 0, None, 1.0, ptr(iz[0]), ptr(gw), *[ptr(t) for t in iz[1:]], ptr(x), x.stride(0), H,
+                              ptr(Q), Q.stride(0), ptr(D), D.stride(0), stream()) == 0
+    Q1, D1 = moe.q8_quantize(x)
+    q, d = host(Q), host(D)
+    assert np.array_equal(q[:M, :H], host(Q1)) and np.array_equal(d[:M, :H // 32], host(D1))
+    assert (q[:M, H:] == 77).all() and (q[M] == 77).all() and (d[:M, H // 32:] == -7.0).all() and (d[M] == -7.0).all()
+    rid, rgw = orc.router_topk(host(lg), k)
+    cnt, off, xrow, where = orc.moe_sort(rid, E)
+    assert np.array_equal(host(iz[0]).reshape(M, k), rid) and np.allclose(host(gw).reshape(M, k), rgw, rtol=2e-6, atol=1e-7)
+    for got, want in zip(iz[1:5], (cnt, off, xrow, where)):
+        assert np.array_equal(host(got), want)
