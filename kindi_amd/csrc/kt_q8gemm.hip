@@ -17,8 +17,8 @@
 
    Measured on MI355X (128 experts, 6 picks, even router, up [1856 x 2688] / down [2688 x 1856], against k_q8_mma): 96
    entries an expert 1003 / 981 -> 394 / 372 us, 24: 309 / 302 -> 174 / 157, 12: 166 / 168 -> 152 / 151 (678 MB of weights: 4.5 TB/s).
-   The refill goes out only where another slice or pass of the block follows: with one after the last (KS + 1 slices read for
-   KS) 12 entries took 156 / 167 us, 24: 178 / 176. At long lists the SIMDs bound it: a unit of a tile takes
+   The refill after a block's last slice reads an empty buffer: with the first slice read again there (KS + 1 slices for KS) 12
+   entries took 156 / 167 us, 24: 178 / 176. At long lists the SIMDs bound it: a unit of a tile takes
    about 37 vector and 1.5 matrix instructions, and 2 waves a SIMD (253 registers) issue at most one vector instruction
    each about every 4 cycles; without any global load 96 entries take 296 us. */
 #include <type_traits>
@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
   const uint32_t OOB = 0x80000000u;
   const kt_v4i rx = kt_dma_rsrc(xq, (uint32_t)nrows * (uint32_t)ldq);
   const kt_v4i rs = kt_dma_rsrc(xd, (uint32_t)nrows * (uint32_t)ldd * 4u);
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)wbuf, (short)0, R8 * NU * 272, 0x00020000);
+  __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)wbuf, (short)0, R8 * NU * 272, 0x00020000);
   const uint32_t la = kt_dma_lds(L.a), lx = kt_dma_lds(L.x);
   const int ao = n * 512 + ((h ^ (n & 15)) << 4), xo = n * 64 + ((2 * h) ^ ((n >> 2) & 3)) * 16;   /* this lane's operands */
   const uint32_t wb = rg < R8 ? (uint32_t)(rg * NU * 16 + (row & 7)) * 16u : OOB;
@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
   };
   KT_QG_C(qg_ldw(rw, c_, 0, S / KS, S, ncl, h, wf, wl, db, wq[0][c_], wq[1][c_], hq[c_]))
   /* tile tt of the pass, slice from s0: its activations and token scales into stage st */
-  auto issue = [&](int st, int tt, int s0, int ns, int nt){
+  auto issue = [&](int st, int tt, int s0, int ns){
     /* activations: instruction i = rows 2 i, 2 i + 1; lane: row 2 i + lane / 32, chunk position lane % 32 */
 #pragma unroll
     for(int q = 0; q < 4; ++q){
@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
       L.rd[tid] = ok ? (uint32_t)r * (uint32_t)ldd * 4u : OOB;
     }
     __syncthreads();
-    issue(0, 0, 0, S / KS, nt);
+    issue(0, 0, 0, S / KS);
     int st = 0;
     bool refilled = false;                                         /* uniform */
     for(int k = 0; k < KS; ++k){
@@ -208,10 +208,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
         if(refilled && !DBG) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(KT_QG_LOADS) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        /* the weights' last tile refills them, for the next slice or the first one of the block's next pass */
-        refilled = tt + 1 == T && (k + 1 < KS || t0 + t_st < t_hi);
-        if(tt + 1 < T) issue(st ^ 1, tt + 1, s0, ns, nt);
-        else if(k + 1 < KS) issue(st ^ 1, 0, sn, nsn, nt);
+        refilled = tt + 1 == T;
+        if(!refilled) issue(st ^ 1, tt + 1, s0, ns);
+        else if(k + 1 < KS) issue(st ^ 1, 0, sn, nsn);
+        /* the refill after the block's last slice has nothing to fetch: an empty buffer's loads make no memory access */
+        if(k + 1 == KS && t0 + t_st >= t_hi) rw = __builtin_amdgcn_make_buffer_rsrc((void*)wbuf, (short)0, 0, 0x00020000);
         tile(refilled, st, tt, k, s0, ns, sn, nsn, t0);
         st ^= 1;
       }
