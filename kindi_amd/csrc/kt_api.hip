@@ -26,7 +26,7 @@ template <bool DBG>
 __global__ void k_gemv_pair(const KtGemvArgs, const int8_t*, const float*, const int*, int32_t*, int);
 template <int NT, bool DBG, int LB>
 __global__ void k_gemv_mma(const KtGemvArgs, const int8_t*, const float*, int32_t*, int);
-template <bool DBG, int KQ, bool MS>
+template <bool DBG, int KQ, bool MS, bool LT>
 __global__ void k_gemv_m16(const KtGemvArgs, const int8_t*, const float*, const int*, int32_t*, int);
 template <bool GRP, bool DBG, bool MS>
 __global__ void k_q8_mma(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
@@ -124,6 +124,33 @@ static bool kt_use_mma(const KtGemvArgs& a){
   return w >= KT_MMA_W2;
 }
 
+/* the current device's CU count, queried once per device */
+static int kt_cu_count(int* cus){
+  static int cache[64];
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if(e != hipSuccess) return (int)e;
+  if(dev < 0 || dev >= 64) return KT_INVALID;
+  if(!cache[dev]){
+    int n = 0;
+    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    if(e != hipSuccess) return (int)e;
+    cache[dev] = n;
+  }
+  *cus = cache[dev];
+  return 0;
+}
+
+/* k_gemv_m16's activations straight into the operand (not through LDS): few rows in a pass, or few loads a CU (at most a
+   tile a CU, and slices times rows up to 16). MI355X, us straight / through LDS: 5 rows [2048 x 6144] 5.6 / 5.8, [12288 x 4096]
+   6.7 / 6.9, [4096 x 12288] 8.8 / 8.9, 8 rows 6.0 / 5.9, 7.2 / 7.0, 9.6 / 9.2; 3 / 5 rows [17408 x 5120] 11.2 / 11.6 against 11.3 / 11.4 (more
+   tiles than 2 a CU and 3 slices or more: up to 3 rows); 16 rows [2048 x 2048] 4.0 / 4.2, [512 x 2048] 3.8 / 4.1, 8 and 12 rows [1024
+   x 4096] 4.8 / 4.9 and 5.1 / 4.9 */
+static bool kt_m16_direct(int tiles, int passes, int ks, int M, int cus){
+  const int rows = M < 16 ? M : 16;
+  return rows <= (tiles > 2 * cus && ks > 2 ? 3 : 5) || (tiles * passes <= cus && ks * rows <= 16);
+}
+
 static int kt_launch_mma(KtGemvArgs a, const int8_t* xq, const float* xs, const int* xa, int32_t* dbg,
                          hipStream_t s){
   const int ks = kt_kslices(a.NU);
@@ -131,6 +158,10 @@ static int kt_launch_mma(KtGemvArgs a, const int8_t* xq, const float* xs, const 
   for(int i = 0; i < a.nmat; ++i){ a.mat[i].pad = tiles; tiles += (kt_r8(a.mat[i].R) + 3) / 4; }
   const dim3 grid(tiles, (a.M + 15) / 16), block(64 * ks);
   const size_t lds = (size_t)ks * 16 * 32 * 4 + (size_t)ks * 256 * 4;        /* slice sums, XS */
+  int cus = 0;
+  const int ec = kt_cu_count(&cus);
+  if(ec) return ec;
+  const bool direct = kt_m16_direct(tiles, (int)grid.y, ks, a.M, cus);
   bool off32 = (long long)a.M * a.ldxs * 4 < (1ll << 31);      /* k_gemv_m16 reads through 32-bit buffer offsets */
   for(int i = 0; i < a.nmat; ++i) off32 = off32 && kt_code_bytes(a.mat[i].R, a.NU) < (1ull << 31);
   if(ks <= 10 && off32){
@@ -148,24 +179,21 @@ static int kt_launch_mma(KtGemvArgs a, const int8_t* xq, const float* xs, const 
          13.8 / 14.2 / 15.0 -> 12.8 / 13.0 / 14.2 us; slower at 16 tokens, 17.35 -> 17.75 us, so up to 8 tokens) */
       const size_t lq = (size_t)ks * 4 * 16 * 32 * 4 + (size_t)G * 4 * 512 * 4;   /* pair sums, XS + XA a wave */
       const dim3 bq(256 * G);
-      if(ms){
-        if(dbg) KT_LAUNCH((k_gemv_m16<true, 4, true>), grid, bq, lq, s, a, xq, xs, xa, dbg, ks);
-        else KT_LAUNCH((k_gemv_m16<false, 4, true>), grid, bq, lq, s, a, xq, xs, xa, dbg, ks);
-      } else {
-        if(dbg) KT_LAUNCH((k_gemv_m16<true, 4, false>), grid, bq, lq, s, a, xq, xs, xa, dbg, ks);
-        else KT_LAUNCH((k_gemv_m16<false, 4, false>), grid, bq, lq, s, a, xq, xs, xa, dbg, ks);
-      }
+#define KT_M16(KQ, MS, LT, B, LDS) do { \
+        if(dbg) KT_LAUNCH((k_gemv_m16<true, KQ, MS, LT>), grid, B, LDS, s, a, xq, xs, xa, dbg, ks); \
+        else KT_LAUNCH((k_gemv_m16<false, KQ, MS, LT>), grid, B, LDS, s, a, xq, xs, xa, dbg, ks); } while(0)
+      if(ms){ if(direct) KT_M16(4, true, false, bq, lq); else KT_M16(4, true, true, bq, lq); }
+      else { if(direct) KT_M16(4, false, false, bq, lq); else KT_M16(4, false, true, bq, lq); }
     } else if(ks > 4 && a.M > KT_M16Q_MSM && (long long)tiles * grid.y * 16 <= KT_M16H_WAVES){
       /* above 8 tokens: the k-lanes of a slice over 2 waves, 8 slice groups (16 waves a block; measured on MI355X,
          27B-class down at 16 tokens 17.41 -> 17.19 us against whole-slice waves) */
       const size_t lh = (size_t)ks * 2 * 16 * 32 * 4 + (size_t)16 * 512 * 4;
-      if(dbg) KT_LAUNCH((k_gemv_m16<true, 2, true>), grid, dim3(1024), lh, s, a, xq, xs, xa, dbg, ks);
-      else KT_LAUNCH((k_gemv_m16<false, 2, true>), grid, dim3(1024), lh, s, a, xq, xs, xa, dbg, ks);
+      KT_M16(2, true, true, dim3(1024), lh);
     } else {
       const size_t lds16 = lds + (size_t)ks * 256 * 4;                      /* + XA */
-      if(dbg) KT_LAUNCH((k_gemv_m16<true, 1, false>), grid, block, lds16, s, a, xq, xs, xa, dbg, ks);
-      else KT_LAUNCH((k_gemv_m16<false, 1, false>), grid, block, lds16, s, a, xq, xs, xa, dbg, ks);
+      if(direct) KT_M16(1, false, false, block, lds16); else KT_M16(1, false, true, block, lds16);
     }
+#undef KT_M16
   } else {
     /* above 10 slices, or buffers past 32-bit offsets: 32x32x32 tiles, the 1024-thread bound (activations loaded in
        place, 124 VGPRs) */
@@ -426,23 +454,6 @@ hipError_t kt_rec_push(const void* fn, dim3 g, dim3 b, size_t lds, int n, const 
   L.shmem = (unsigned)lds;
   L.nargs = n;
   return hipSuccess;
-}
-
-/* the current device's CU count, queried once per device */
-static int kt_cu_count(int* cus){
-  static int cache[64];
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if(e != hipSuccess) return (int)e;
-  if(dev < 0 || dev >= 64) return KT_INVALID;
-  if(!cache[dev]){
-    int n = 0;
-    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    if(e != hipSuccess) return (int)e;
-    cache[dev] = n;
-  }
-  *cus = cache[dev];
-  return 0;
 }
 
 extern "C" {

@@ -241,7 +241,7 @@ __device__ __forceinline__ kt_v4i km_digits16(uint32_t w){
 #else
 #define KT_M16TS(k) do {} while(0)
 #endif
-template <bool DBG, int KQ, bool MS>
+template <bool DBG, int KQ, bool MS, bool LT>   /* LT: activations through LDS */
 __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvArgs a, const int8_t* __restrict__ xq,
                                                   const float* __restrict__ xs, const int* __restrict__ xav,
                                                   int32_t* __restrict__ dbg, int KS){
@@ -283,14 +283,15 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
   float* xsl = (float*)(kt_lds + (size_t)KS * KQ * NT * 32 * 4) + (size_t)wvi * 512;
   int* xal = (int*)(xsl + 256);
   /* activations through a buffer resource over the M token rows (lanes past the pass's tokens: past the range,
-     zeros without a memory access). A load has 4 neighbouring lanes on one row: in the operand's own order (16 lanes on 16
-     rows) it holds the address unit 27.5 ns, so 7.2 (measured a CU): MI355X, 16 tokens, 27B gate/up 25.6 -> 20.4 us, down 17.5 -> 15.0,
-     q/k/v 8.0 -> 7.3, o 7.2 -> 6.6, with the token scales' loads regrouped the same way. The rows then go through this wave's slot of red (2 KB,
-     its slice sums' place, free until they are written) into the operand order: row r of 128 bytes, 16-byte chunk c at
-     position c ^ f(r), f the bits of (r >> 1) & 7 rotated so that neither the 4-row writes nor the 16-row reads share banks */
+     zeros without a memory access). !LT: straight into the operand, 16 lanes on 16 rows, which holds the address unit up
+     to 27.5 ns a load (measured a CU). LT: 4 neighbouring lanes on one row, 7.2 ns; MI355X, 16 tokens, 27B gate/up 25.6 ->
+     20.4 us, down 17.5 -> 15.0, q/k/v 8.0 -> 7.3, o 7.2 -> 6.6, with the token scales' loads regrouped the same way. The rows
+     then go through this wave's slot of red (2 KB, its slice sums' place, free until they are written) into the operand order: row
+     r of 128 bytes, 16-byte chunk c at position c ^ f(r), f the bits of (r >> 1) & 7 rotated so that neither the 4-row writes
+     nor the 16-row reads share banks. That trip adds 0.2 us to a launch, so few rows load straight (kt_m16_direct) */
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)xq, (short)0, a.M * a.ldq, 0x00020000);
-  const int lt = lane >> 2;
-  const uint32_t xoff = lt < nt ? (uint32_t)((t0 + lt) * a.ldq + 16 * (lane & 3)) : (1u << 30);
+  const int lt = LT ? lane >> 2 : n;
+  const uint32_t xoff = lt < nt ? (uint32_t)((t0 + lt) * a.ldq + 16 * (LT ? lane & 3 : g)) : (1u << 30);
   auto km_f = [](int r){ const int s3 = (r >> 1) & 7; return (s3 & 1) << 2 | s3 >> 1; };
   const int awr = lt * 128 + (((lane & 3) ^ km_f(lt)) << 4), ard = n * 128 + ((g ^ km_f(n)) << 4);
   for(int it = 0, ks = sg; MS ? ks < KS : it < 1; ++it, ks += G){                /* !MS: one slice a wave */
@@ -303,7 +304,7 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
   int xdst[NI];
 #pragma unroll
   for(int i = 0; i < NI; ++i){
-    const int idx = lane + 64 * i, un = idx % (2 * CW), tl = idx / (2 * CW);
+    const int idx = lane + 64 * i, un = LT ? idx % (2 * CW) : idx >> 4, tl = LT ? idx / (2 * CW) : idx & 15;
     const int j = un / CW, c = cb + un % CW;                     /* the wave's units: CW k-lanes, 2 steps */
     const int u = (s_lo + j) * KT_KL + c;
     const int t = t0 + tl < a.M ? t0 + tl : t0;
@@ -366,11 +367,15 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
         unsigned w0 = wq[j][cc].x, w1 = wq[j][cc].y, w2 = wq[j][cc].z, w3 = wq[j][cc].w;
         km_swap32(w0, w2); km_swap32(w1, w3);
         km_swap16(w0, w1); km_swap16(w2, w3);
-        uint8_t* ab = kt_lds + (size_t)(ks * KQ + q) * 2048;       /* chunks 0 - 3 of half 0, 4 - 7 of half 1 */
-        *(kt_v4i*)(ab + awr) = kt_v4i{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w};
-        *(kt_v4i*)(ab + (awr ^ 64)) = kt_v4i{(int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
-        kt_wave_sync();
-        const kt_v4i A0 = *(const kt_v4i*)(ab + ard), A1 = *(const kt_v4i*)(ab + (ard ^ 64));
+        kt_v4i A0 = {(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w}, A1 = {(int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+        if constexpr(LT){
+          uint8_t* ab = kt_lds + (size_t)(ks * KQ + q) * 2048;     /* chunks 0 - 3 of half 0, 4 - 7 of half 1 */
+          *(kt_v4i*)(ab + awr) = A0;
+          *(kt_v4i*)(ab + (awr ^ 64)) = A1;
+          kt_wave_sync();
+          A0 = *(const kt_v4i*)(ab + ard);
+          A1 = *(const kt_v4i*)(ab + (ard ^ 64));
+        }
         /* both chains start from -XA of tokens 4 g .. + 3 (staged negated), so they end at v = sum d q - XA */
         const int4 xa4 = *(const int4*)(xal + (j * 8 + c) * 16 + 4 * g);
         const kt_v4i cx = {xa4.x, xa4.y, xa4.z, xa4.w};
@@ -415,7 +420,7 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
   KT_M16TS(2);
   /* slices in order (KQ = 4: the pair sums of a slice first, (p0 + p1) + (p2 + p3)) */
   /* a lane's 8 sums as two float4 at [slice][quarter][half][lane]: 16-byte LDS accesses, conflict free */
-  kt_wave_sync();                                                /* the slot's last activations are read */
+  if constexpr(LT) kt_wave_sync();                               /* the slot's last activations are read */
   {
     float4* r4 = (float4*)red + (size_t)(ks * KQ + q) * 128 + lane;
     r4[0] = make_float4(part[0], part[1], part[2], part[3]);
@@ -460,10 +465,11 @@ __global__ void __launch_bounds__(KQ == 1 ? 640 : 1024) k_gemv_m16(const KtGemvA
   }
 }
 
-#define KM16_INST(DBG, KQ, MS) template __global__ void k_gemv_m16<DBG, KQ, MS>(const KtGemvArgs, const int8_t*, \
-    const float*, const int*, int32_t*, int);
-KM16_INST(false, 1, false) KM16_INST(true, 1, false) KM16_INST(false, 4, false) KM16_INST(true, 4, false)
-KM16_INST(false, 4, true) KM16_INST(true, 4, true) KM16_INST(false, 2, true) KM16_INST(true, 2, true)
+#define KM16_INST(KQ, MS, LT) template __global__ void k_gemv_m16<false, KQ, MS, LT>(const KtGemvArgs, const int8_t*, \
+    const float*, const int*, int32_t*, int); template __global__ void k_gemv_m16<true, KQ, MS, LT>(const KtGemvArgs, \
+    const int8_t*, const float*, const int*, int32_t*, int);
+KM16_INST(1, false, false) KM16_INST(1, false, true) KM16_INST(4, false, false) KM16_INST(4, false, true)
+KM16_INST(4, true, false) KM16_INST(4, true, true) KM16_INST(2, true, true)
 #undef KM16_INST
 
 /* ------------------------------------------------------------------ q8_0 on the matrix cores

@@ -54,6 +54,34 @@ def test_gemm_routes(R, C, M, route, per_row):
     assert np.array_equal(host(wide[:, :R]), want) and bool((wide[:, R:] == -7.0).all())
 
 
+# the 16-token decode product with its activations straight into the operand and through LDS: both sides of 5 rows (3 above 2
+# tiles a CU of 3 slices or more) and of slices x rows 16 at a tile a CU; whole slices, slices over 4 waves, more slices than 4
+# groups, over 2 waves; a second pass of one token; the two-row form
+@pytest.mark.parametrize("R,C,Ms", [(40, 384, (3, 5, 6, 15, 16, 17)), (100, 2048, (4, 16, 17)), (8200, 2048, (5, 6)), (1000, 4096, (8, 9)), (520, 6144, (5, 6)),
+                                    (16648, 5120, (3, 4)), (136, 9216, (5, 6, 9, 17)), (100, 12288, (3, 5, 6, 8, 9, 16))])
+@pytest.mark.parametrize("hp", [False, True])
+def test_decode_rows_either_way(R, C, Ms, hp):
+    from kindi_amd import linear
+    dig, bc, dpm = tern_case(R, C, R + C)
+    L = linear.Linear({"w": linear.TernaryMatrix(bc, dpm, R, C)})
+    X = dev(rng(C).normal(0, 1, (max(Ms), C)).astype(np.float32))
+    one = torch.empty((max(Ms), R), device="cuda")
+    for i in range(max(Ms)):                                              # a token at a time: the same bits in any company
+        L.gemv_q(["w"], linear.quantize(X[i:i + 1], hp=hp), [one[i:i + 1]])
+    for M in Ms:
+        say("decode rows", R, C, M, hp)
+        act = linear.quantize(X[:M], hp=hp)
+        Y = torch.empty((M, R), device="cuda")
+        L.gemv_q(["w"], act, [Y])
+        assert torch.equal(Y, one[:M]), M
+        rows = act.XQ.shape[0]
+        if rows * R * C <= 1 << 25:
+            dbg = torch.empty((rows, R, C // 128), dtype=torch.int32, device="cuda")
+            Y2 = torch.empty((M, R), device="cuda")
+            L.gemv_q(["w"], act, [Y2], dbg=dbg)
+            assert torch.equal(Y2, one[:M]) and np.array_equal(host(dbg), orc.tern_acc(bc, R, C, host(act.XQ))), M
+
+
 @pytest.mark.parametrize("R,M,route", [(256, 64, "split"), (8200, 70, "one"), (8200, 400, "two")])
 def test_gemm_scale_extremes(R, M, route):
     """token scales whose product with a row scale is subnormal, overflows, or is not a number: the element scale is
