@@ -467,6 +467,19 @@ static bool kf_overlap(const float* p, int ldp, const float* q, int ldq, int M, 
   const uintptr_t q0 = (uintptr_t)q, q1 = q0 + ((size_t)(M - 1) * ldq + C) * 4;
   return p0 < q1 && q0 < p1;
 }
+/* ... and rows that meet: [a | b | xo] rows of one buffer lie between one another without doing so */
+static bool kf_rows_meet(const float* p, int ldp, const float* q, int ldq, int M, int C){
+  if(!kf_overlap(p, ldp, q, ldq, M, C)) return false;
+  const long long d = ((long long)(intptr_t)p - (long long)(intptr_t)q) / 4;        /* floats from q to p */
+  for(int i = 0; i < M; ++i){                                       /* row i of p against the last row of q that starts before its end */
+    const long long e = d + (long long)i * ldp;
+    if(e + C <= 0) continue;
+    const long long j = (e + C - 1) / ldq;
+    if((j < M ? j : M - 1) * ldq + C > e) return true;
+    if(ldp == ldq && j < M) return false;                           /* equal strides: the other rows lie the same way */
+  }
+  return false;
+}
 
 hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
   /* rmsfold over chunks of a row: every chunk's block reads the whole row (x and the parts, for the norm) while it
@@ -478,8 +491,8 @@ hipError_t kt_fold_launch(int mode, const KtFoldArgs& a, int M, hipStream_t s){
       || kf_overlap(a.xn, a.ldxn, a.r, a.ldr, M, np * a.C) || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, np * a.C))));
   /* smfold's grouped-head order reads other chunks' columns (with one key group, nk 1, it is the plain order): where xo lies
      over an input, a block takes the row, its inputs in LDS before an output is written, at any number of tokens */
-  const bool turned = mode == 2 && a.rep > 1 && a.nk > 1 && (kf_overlap(a.xo, a.ldxo, a.x, a.ldx, M, a.C)
-                      || kf_overlap(a.xo, a.ldxo, a.r, a.ldr, M, a.C));
+  const bool turned = mode == 2 && a.rep > 1 && a.nk > 1 && (kf_rows_meet(a.xo, a.ldxo, a.x, a.ldx, M, a.C)
+                      || kf_rows_meet(a.xo, a.ldxo, a.r, a.ldr, M, a.C));
   if(turned && a.C > KF_ROW_MAX) return hipErrorInvalidValue;
   const bool narrow = a.C <= KF_NARROW && (mode == 0 || (mode == 2 && a.C == a.HB));
   if((M > KF_FEW || alias || turned) && !narrow){

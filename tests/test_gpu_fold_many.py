@@ -131,3 +131,24 @@ def test_smfold_in_place_refused_past_lds():
         lin.smfold(a, b, sg, 512, perm=(128, 144, 2), xo=a)
     lin.smfold(a, b, sg, 512, perm=(128, 144, 2), xo=torch.empty_like(a))       # not in place, and the plain order: taken
     lin.smfold(a, b, sg, 512, perm=(18432, 1, 2), xo=a)
+
+
+# rows of one buffer that lie between one another and do not meet: [a | b | xo] of one stride, and an xo of twice a's stride;
+# widths that LDS holds and wider
+@pytest.mark.parametrize("C", [6144, 36864])
+@pytest.mark.parametrize("M", [1, 3, 40])
+def test_smfold_between_rows(C, M):
+    from kindi_amd import linear as lin
+    say("smfold between rows", M, C)
+    r = rng(C + M)
+    sg = dev(np.where(r.random(C) < 0.5, -1, 1).astype(np.float32))
+    a, b = (dev(r.standard_normal((M, C)).astype(np.float32)) for _ in range(2))
+    want = torch.empty_like(a)
+    perm = (128, C // 256, 2)
+    a0 = lin.smfold(a, b, sg, 512, perm=perm, xo=want)
+    one = torch.zeros((M, 3 * C), device="cuda")
+    two = torch.zeros((2 * M, 2 * C), device="cuda")
+    for av, xo in ((one[:, :C], one[:, 2 * C:]), (two[:M, :C], two.view(M, 4 * C)[:, C:2 * C])):
+        av.copy_(a)
+        a1 = lin.smfold(av, b, sg, 512, perm=perm, xo=xo)
+        assert _same(xo, want) and _same(av, a) and all(_same(u, v) for u, v in zip((a0.XQ, a0.XS, a0.XA), (a1.XQ, a1.XS, a1.XA)))
