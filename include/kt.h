@@ -200,7 +200,7 @@ int kt_moe_topk_r(const float* logits, int M, int E, int k, int score, const flo
                   float* gw, void* stream);
 int kt_moe_sort(const int* ids, int M, int k, int E, int* cnt, int* off, int* xrow, int* where, int* act, int* nact,
                 void* stream);
-/* kt_moe_route: kt_moe_topk and kt_moe_sort in one launch (one wave; M k <= 64 entries; the same outputs) — the
+/* kt_moe_route: kt_moe_topk and kt_moe_sort in one launch (one block; M k <= 64 entries; the same outputs) — the
    router and list building around lt_router_topk (lightning.cu:414-468) and lt_moe_lists (lightning.cu:1318-1349);
    with x non-NULL, the same launch also writes kt_q8_quant(x, act = 0) into Q / D (H % 32 == 0). */
 int kt_moe_route(const float* logits, int M, int E, int k, int* ids, float* gw, int* cnt, int* off, int* xrow,

@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(64 * PF_NW) __attribute__((amdgpu_waves_per_eu
   auto group = [&](int g, int q){
     /* this wave's DMAs of group g have landed when at most the later groups' are in flight (loads retire in order);
        after the barrier every wave's have, and the stage of group g - 1 is no longer read */
-    if(DBG || g + NS - 2 >= NG || NS == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if(DBG || g + NS - 2 >= NG) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(L::DMA * (NS - 2)) : "memory");
     __syncthreads();
     if(g + NS - 1 < NG) issue(g + NS - 1, (q + NS - 1) % NS);

@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(64 * NW) k_tern_gemm_ks(const uint32_t* __rest
     }
   };
   /* round j from stage q: after the barrier its values are there and the stage of round j - 1 is free. Its groups are
-     applied in order to this thread's outputs (tokens 8 w + 4 h .. + 3, row n) while the next round's values are made */
+     applied in order to this thread's outputs (tokens tok0 .. + EPT - 1 of the tile, row n) while the next round's values are made */
   auto round = [&](int j, int q){
     __syncthreads();
     float v[NW][EPT], s[NW][EPT];

@@ -3,8 +3,10 @@ cross-compiles here).
 
 - No kernel uses scratch (private segment) apart from the listed ones: the debug instantiations (int32 unit values
   written out for the tests).
-- The decode product at 8-32 tokens and both prefill kernels read global memory only through buffer resources that
-  span exactly their buffers, so an out-of-range offset reads zeros and cannot fault.
+- The decode product at 3-32 tokens and the prefill kernels on packed trits read global memory only through buffer resources
+  that span exactly their buffers, so an out-of-range offset reads zeros and cannot fault; the q8_0 product at many tokens
+  reads its weights, activations and scales so (its list tables, 4 bytes an entry, directly).
+- The prefill kernels wait for their DMAs by count: the counts they wait with are the DMAs they issue.
 - No kernel writes through the scalar data cache.
 """
 import os
@@ -47,7 +49,7 @@ def _kernels(text):
             name = m.group(1)
             body = []
             for l2 in lines[i + 1:]:
-                if l2.strip().startswith("s_endpgm"):
+                if l2.startswith((".Lfunc_end", "\t.section")):         # past every s_endpgm: a kernel may return early
                     break
                 body.append(l2.strip())
             out[name] = [body, None]
@@ -62,8 +64,7 @@ def _kernels(text):
 
 
 SCRATCH_OK = {"k_gemv_flat1<0, 1, true, false>", "k_gemv_pair<true>", "k_q8_mma<false, true, false>",
-              "k_q8_mma<true, true, false>", "k_tern_gemm<true, false>", "k_tern_gemm<true, true>",
-              "k_tern_gemm_rs1<4, 2, 3, true>", "k_tern_gemm8<true>", "k_gemv_m16<true, 2, true, true>"}
+              "k_q8_mma<true, true, false>", "k_tern_gemm8<true>", "k_gemv_m16<true, 2, true, true>"}
 
 
 def _demangle(names):
@@ -93,7 +94,7 @@ def _ops(body):
     return [l.split()[0] for l in body if l and not l.startswith((".", ";")) and not l.endswith(":")]
 
 
-@pytest.mark.parametrize("src,pat", [("kt_mma.hip", "k_gemv_m16"), ("kt_prefill.hip", "k_tern_gemm")])
+@pytest.mark.parametrize("src,pat", [("kt_mma.hip", "k_gemv_m16"), ("kt_prefill.hip", "k_tern_gemm_w"), ("kt_prompt.hip", "k_tern_gemm_ks")])
 def test_reads_through_buffer_resources(asm, src, pat):
     ks = {n: b for n, (b, _) in _kernels(asm[src]).items() if pat in n and b}
     assert ks, pat
@@ -102,6 +103,46 @@ def test_reads_through_buffer_resources(asm, src, pat):
         flat = [o for o in ops if o.startswith(("global_load", "flat_load", "global_atomic", "flat_atomic"))]
         assert not flat, (name, flat[:5])
         assert any(o.startswith("buffer_load") for o in ops), name
+
+
+def test_q8_gemm_reads(asm):
+    """k_q8_gemm: dense, everything through buffer resources; grouped, the list tables (single words) beside them"""
+    ks = {n: b for n, (b, _) in _kernels(asm["kt_q8gemm.hip"]).items() if "k_q8_gemm" in n and b}
+    assert len(ks) == 4
+    for name, body in ks.items():
+        ops = _ops(body)
+        flat = {o for o in ops if o.startswith(("global_load", "flat_load", "global_atomic", "flat_atomic"))}
+        assert flat <= ({"global_load_dword"} if "ILb1E" in name else set()), (name, flat)
+        assert sum(o.startswith("buffer_load") for o in ops) > 24, name
+
+
+# the DMAs a wave issues for one stage: k_tern_gemm_w<T>: T of activations, packed trits, row scales (and token scales without
+# RS); k_tern_gemm_ks: 4, 1, 1 (and 1)
+@pytest.mark.parametrize("src,pat,dmas,last", [("kt_prefill.hip", r"k_tern_gemm_wILi(\d)ELb(\d)ELb0E", lambda t, rs: t + 3 - rs, lambda t: 16 * t),
+                                          ("kt_prompt.hip", r"k_tern_gemm_ksILi(\d)ELb(\d)ELb0E", lambda nw, rs: 7 - rs, lambda nw: 16 // nw)])
+def test_dma_waits_are_counted(asm, src, pat, dmas, last):
+    """loads retire in order, so a wait for all but n leaves exactly the last n in flight: n is the DMAs of one stage, each
+    stage between two barriers issues that many or none, and the only other loads are the outputs' token scales at the end (RS)"""
+    seen = 0
+    for name, (body, _) in _kernels(asm[src]).items():
+        m = re.search(pat, name)
+        if not m or not body:
+            continue
+        seen += 1
+        v, rs = int(m.group(1)), int(m.group(2))
+        n = dmas(v, rs)
+        lds = [i for i, l in enumerate(body) if l.startswith("buffer_load") and l.endswith(" lds")]
+        other = [i for i, l in enumerate(body) if re.match(r"(buffer|global|flat|scratch)_load", l) and i not in lds]
+        assert lds and len(lds) % n == 0 and len(other) == (last(v) if rs else 0), (name, len(lds), len(other), n)
+        waits = {int(w) for w in re.findall(r"s_waitcnt vmcnt\((\d+)\)", "\n".join(body))}
+        assert waits == {0, n} or waits == {n}, (name, waits, n)
+        run = 0
+        for l in body + ["s_barrier"]:
+            if l.startswith(("s_barrier", "s_cbranch", "s_branch")) or l.endswith(":"):
+                assert run % n == 0, (name, run, n)
+                run = 0
+            run += l.startswith("buffer_load") and l.endswith(" lds")
+    assert seen == 4
 
 
 def test_no_scalar_cache_writes(asm):
