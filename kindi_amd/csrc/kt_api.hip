@@ -739,17 +739,25 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
      - the matrix cores with a K slice a wave (k_q8_mma, up to 8 slices) from 9 tokens, from 5 on 2^22 weights, from 3 on
        2^25: [2688 x 1856] at 4 / 5 tokens 6.4 against 7.4 / 8.3 -> 7.3 us, [8192 x 4096] at 3 tokens 14.2 -> 11.5,
        [1024 x 1024] at 5 / 10 tokens 6.1 against 6.8 / 8.1 -> 6.9;
-     - k_q8_gemm above 12 (tile of 32 rows, pass of 16 tokens) pairs a CU: [8192 x 4096] at 176 tokens (11 pairs) 49 against 56
-       us, at 224 (14) 59 -> 56, at 288 (18) 72 -> 61; [4096 x 2688] at 336 (10.5) 41 against 42, at 448 (14) 50 -> 42; and from 64
-       tokens where the rows have more than 8 slices: [4096 x 8192] at 50 / 100 tokens 117 / 217 against 98 / 99 us,
-       [1024 x 5120] 42 / 76 against 63 / 63;
+     - k_q8_gemm (above 16 tokens) above ks + 4 (tile of 32 rows, pass of 16 tokens) pairs a CU, 3 where a row is one slice. k_q8_gemm's time
+       goes with the steps of a row, k_q8_mma's with the pairs and little with the slices. Pairs, us on k_q8_mma / k_q8_gemm: ks 1
+       [8192 x 512] 3 11.0 / 10.3, 4 13.7 / 10.4; ks 2 [8192 x 1024] 4 15.2 / 16.6, 7 23.4 / 17.0, [16384 x 1024] 6 14.3 / 16.8; ks 3 [8192 x
+       1536] 5 19.1 / 23.1, 8 27.6 / 23.7; ks 4 [8192 x 2048] 7 25.8 / 28.9, 9 31.7 / 29.1; ks 5 [8192 x 2560] 9 34.4 / 35.4, 10 37.4 /
+       35.1; ks 6 [8192 x 2688] 10 37.8 / 40.9, 11 41.2 / 40.8; ks 8 [8192 x 4096] 11 49 / 56, 14 59 / 56;
+     - above 8 slices k_q8_gemm against the v_dot4 kernel, whose time goes with tokens times its rounds of row groups over the
+       CUs, from 88 of them, from 50 where the tokens are one tile of 32: [512 .. 2048 x 5120] (1) at 80 / 88 tokens 61.6 .. 65.5 / 67.4 ..
+       71.2 against 64.2, [2048 x 8192] 92 / 101 against 99.8; [4096 x 5120] (2) at 24 / 32 tokens 41.5 / 52.8 against 37.4, 40 / 48
+       64.6 / 75.7 against 63.5, [4096 x 8192] 24 57.4 against 57.0, 40 / 48 90.9 / 107 against 98.8; [8192 x 5120] (4) at 24 78.5
+       against 37.6;
      - the v_dot4 kernel else. */
   int cus = 0;
   const int ec = kt_cu_count(&cus);
   if(ec) return ec;
   const int tiles = (kt_r8(R) + 3) / 4, np = M / 16 + (M % 16 ? 1 : 0);
   const long long nw = (long long)R * C;
-  if((ks <= KT_Q8_MMA_KS ? (long long)tiles * np > 12ll * cus : M >= 64) && kt_q8_gemm_takes(NB)
+  const int rounds = (kt_r8(R) + cus - 1) / cus;
+  if((ks <= KT_Q8_MMA_KS ? M > 16 && (long long)tiles * np > (ks == 1 ? 3ll : ks + 4ll) * cus
+                         : M >= 9 && (long long)M * rounds >= (M > 32 ? 88 : 50)) && kt_q8_gemm_takes(NB)
      && (long long)M * ldq < (1ll << 31)
      && (long long)M * ldd * 4 < (1ll << 31) && (long long)kt_r8(R) * NB * 272 < (1ll << 31) && (M + 63) / 64 <= 65535){
     const dim3 grid((R + 127) / 128, (M + 63) / 64);
