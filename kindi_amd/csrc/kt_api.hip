@@ -28,7 +28,7 @@ template <int NT, bool DBG, int LB>
 __global__ void k_gemv_mma(const KtGemvArgs, const int8_t*, const float*, int32_t*, int);
 template <bool DBG, int KQ, bool MS, bool LT>
 __global__ void k_gemv_m16(const KtGemvArgs, const int8_t*, const float*, const int*, int32_t*, int);
-template <bool GRP, bool DBG, bool MS>
+template <bool GRP, bool DBG, bool MS, bool LT>
 __global__ void k_q8_mma(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
 template <bool GRP, bool DBG>
 __global__ void k_q8_gemm(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int, int);
@@ -772,8 +772,8 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
     const int want = (cus + tiles - 1) / tiles, gy = want < np ? want : np;
     const dim3 grid(tiles, gy), block(64 * ks);
     const size_t lds = (size_t)ks * (16 * 32 * 4 + 256 * 4) + (size_t)ks * KT_Q8_MMA_ACT;   /* slice sums, D, activations */
-    if(dbg) KT_LAUNCH((k_q8_mma<false, true, false>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
-    else KT_LAUNCH((k_q8_mma<false, false, false>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
+    if(dbg) KT_LAUNCH((k_q8_mma<false, true, false, true>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
+    else KT_LAUNCH((k_q8_mma<false, false, false, true>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);
     return 0;
   }
   return kt_launch_gemv<KT_FMT_Q8>(a, kt_r8(R), Q, D, NULL, dbg, kt_stream(stream));
@@ -874,16 +874,22 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
     const dim3 grid((kt_r8(R) + 3) / 4, ny), block(64 * ks);
     const size_t lds = (size_t)ks * (16 * 32 * 4 + 256 * 4) + (size_t)(ks > 2 ? 2 : ks) * KT_Q8_MMA_ACT;   /* as above */
     const KtGemvArgs da = {};
+    /* activations straight into the operand (not through LDS) at few entries, even router: [2048 x 768] of 128 experts (2 slices) at
+       4 / 6 / 8 56.0 / 57.4 / 59.0 against 57.7 / 60.2 / 62.6 us, [2048 x 4096] of 32 (8) 61.0 / 61.8 / 62.3 against 62.6 / 62.5 / 63.2,
+       [1856 x 2688] of 128 (6) at 5 / 8 135.2 / 143.2 against 135.3 / 141.2; not one slice ([1024 x 512] of 64 10.5 against 10.3) */
+    const bool direct = nentries < (ks == 1 ? 0 : ks == 2 ? 10 : ks <= 6 ? 6 : 9) * (long long)ny;
+#define KT_QM(MS, LT, B) do { \
+      if(dbg) KT_LAUNCH((k_q8_mma<true, true, MS, LT>), grid, B, lds, s, da, a, Q, D, dbg, ks); \
+      else KT_LAUNCH((k_q8_mma<true, false, MS, LT>), grid, B, lds, s, da, a, Q, D, dbg, ks); } while(0)
     if(ks > 2){
       /* two waves a block taking the slices in turn (the same slice sums in the same order): blocks of 2 waves at
          2 waves a SIMD fill every wave slot of a CU, where KS-wave blocks left slots empty (6 slices: 6 of 8) and
          with them weight bytes in flight (measured on MI355X, config 4 M=256: up 223 -> 162 us, down 161 -> 158 us;
          one wave a block 169 / 157, three 185 / 210) */
       const dim3 blk(128);
-      if(dbg) KT_LAUNCH((k_q8_mma<true, true, true>), grid, blk, lds, s, da, a, Q, D, dbg, ks);
-      else KT_LAUNCH((k_q8_mma<true, false, true>), grid, blk, lds, s, da, a, Q, D, dbg, ks);
-    } else if(dbg) KT_LAUNCH((k_q8_mma<true, true, false>), grid, block, lds, s, da, a, Q, D, dbg, ks);
-    else KT_LAUNCH((k_q8_mma<true, false, false>), grid, block, lds, s, da, a, Q, D, dbg, ks);
+      if(direct) KT_QM(true, false, blk); else KT_QM(true, true, blk);
+    } else if(direct) KT_QM(false, false, block); else KT_QM(false, true, block);
+#undef KT_QM
     return 0;
   }
   /* the decode product per (row group, active expert), the expert's list in chunks of up to 4 tokens */

@@ -485,7 +485,7 @@ KM16_INST(4, true, false) KM16_INST(4, true, true) KM16_INST(2, true, true)
    units 8 s + c, the butterfly's tree over c, the slices in order. */
 #define KM_Q8_KS 8                    /* at most 8 K slices (q8_0 C <= 4096): 256 VGPRs a lane */
 #define KM_Q8_ACT (KM_TOK * 512)      /* LDS bytes a wave: a pass's activations of a slice */
-template <bool GRP, bool DBG, bool MS>   /* MS: wave w takes slices w, w + W, ... (W waves a block) */
+template <bool GRP, bool DBG, bool MS, bool LT>   /* MS: wave w takes slices w, w + W, ... (W waves a block); LT: activations through LDS */
 __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, const KtGroupedArgs ga,
                                                           const int8_t* __restrict__ xq, const float* __restrict__ xd,
                                                           int32_t* __restrict__ dbg, int KS){
@@ -531,10 +531,10 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
      tokens (to this wave's LDS region before the products, so the epilogue reads them there), and the activations
      of the 16 units through a buffer resource over the input rows (a token past the pass and a unit past the slice or
      the matrix read at 2^31, past the range, which gives zeros without a memory access; the launcher keeps the rows
-     below 2^31 bytes). Neighbouring lanes are on one row: in the matrix cores' operand order (32 lanes on 16 rows) a load
-     holds the address unit 27.5 ns, so 7.2 (measured a CU). The rows go through LDS: 512 bytes each, 16-byte chunk c of
-     row r at c ^ f(r), f the two bit pairs of r exchanged (neither the 4-row writes nor the 16-row reads share banks). MI355X,
-     dense [8192 x 4096] at 16 / 50 / 100 tokens 13.2 / 25.0 / 40.4 -> 11.5 / 22.0 / 32.8 us, grouped up [1856 x 2688], 128 experts, at
+     below 2^31 bytes). !LT: straight into the operand (32 lanes on 16 rows), which holds the address unit up to 27.5 ns a
+     load (measured a CU). LT: neighbouring lanes on one row, 7.2 ns; the rows then go through LDS: 512 bytes each, 16-byte
+     chunk c of row r at c ^ f(r), f the two bit pairs of r exchanged (neither the 4-row writes nor the 16-row reads share
+     banks). That trip costs what few entries do not repay (kt_q8_grouped has the line). MI355X, dense [8192 x 4096] at 16 / 50 / 100 tokens 13.2 / 25.0 / 40.4 -> 11.5 / 22.0 / 32.8 us, grouped up [1856 x 2688], 128 experts, at
      6 / 9 entries an expert 132 / 156 -> 128 / 149 */
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)xq, (short)0, nrows * ldq, 0x00020000);
   float* xsl = (float*)(kt_lds + (size_t)KS * NT * 32 * 4) + (size_t)wv * 256;
@@ -543,7 +543,8 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
   const int aw = at * 512 + ((ac ^ (at >> 2)) << 4), ax = (at & 3) << 6;
   const int ar = r16 * 512 + ((h ^ ((r16 & 3) << 2) ^ (r16 >> 2)) << 4);
   float xsv[4];
-  uint4 xa[8];
+  uint4 xa[LT ? 8 : 16];
+  const int al = LT ? at : lr;                                   /* the token that this lane loads */
   /* the pass's input rows (the list indirection) first, the loads that need them after */
   int nrq[4], na = 0;
   auto ld_rows = [&](int t0){
@@ -554,7 +555,7 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
       const int pt = p0 + t0 + (tl < nt ? tl : 0);
       nrq[q] = xrow ? xrow[pt] : pt;
     }
-    const int pe = p0 + t0 + (at < nt ? at : 0);
+    const int pe = p0 + t0 + (al < nt ? al : 0);
     na = xrow ? xrow[pe] : pe;
   };
   auto ld_pass = [&](int t0){
@@ -564,11 +565,20 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
       const int u = u0 + r16;
       xsv[q] = xd[(long long)nrq[q] * ldd + (u < NU ? u : 0)];
     }
-    const uint32_t xo = (uint32_t)(na * ldq + u0 * 32 + ac * 16);
+    const uint32_t xo = (uint32_t)(na * ldq + u0 * 32 + (LT ? ac : h) * 16);
+    if constexpr(LT){
 #pragma unroll
-    for(int i = 0; i < 8; ++i)
-      xa[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xr,
-                                 at < nt && 2 * i + (ac >> 1) < nu ? xo + i * 64 : 1u << 31, 0, 0));
+      for(int i = 0; i < 8; ++i)
+        xa[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xr,
+                                   at < nt && 2 * i + (ac >> 1) < nu ? xo + i * 64 : 1u << 31, 0, 0));
+    } else {
+      const uint32_t xl = lr < nt ? xo : 1u << 31;               /* unit 8 j + c of the slice; past it the first one, not used */
+#pragma unroll
+      for(int n = 0; n < 16; ++n){
+        const int u = 8 * (n & 1) + (n >> 1);
+        xa[n] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xr, xl + (u < nu ? u * 32 : 0), 0, 0));
+      }
+    }
   };
   /* the slice's 16 units in k-lane-major order (unconditional: a unit past the slice or the matrix reads offset 0) */
   uint4 wq[2][KT_KL];
@@ -588,12 +598,14 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
   auto compute = [&](int t0){
 #pragma unroll
     for(int q = 0; q < 4; ++q) xsl[r16 * 16 + (lane >> 4) + 4 * q] = xsv[q];
+    if constexpr(LT){
 #pragma unroll
-    for(int i = 0; i < 8; ++i) *(uint4*)(xal + (aw ^ ax ^ (i * 64))) = xa[i];
+      for(int i = 0; i < 8; ++i) *(uint4*)(xal + (aw ^ ax ^ (i * 64))) = xa[i];
+    }
     kt_wave_sync();
     uint4 xn[2];
 #pragma unroll
-    for(int j = 0; j < 2; ++j) xn[j] = *(const uint4*)(xal + ar + 256 * j);
+    for(int j = 0; j < 2; ++j) xn[j] = LT ? *(const uint4*)(xal + ar + 256 * j) : xa[j];
     float part[NE], t01[NE], t23[NE], t45[NE], pend[NE];
 #pragma unroll
     for(int e = 0; e < NE; ++e){ part[e] = 0.0f; t01[e] = 0.0f; t23[e] = 0.0f; t45[e] = 0.0f; pend[e] = 0.0f; }
@@ -604,7 +616,8 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
       for(int e = 0; e < NE; ++e) chain[e] = 0.0f;
       const uint4 xc[2] = {xn[0], xn[1]};
 #pragma unroll
-      for(int j = 0; j < 2; ++j) if(c + 1 < KT_KL) xn[j] = *(const uint4*)(xal + (ar ^ ((c + 1) * 32)) + 256 * j);
+      for(int j = 0; j < 2; ++j)
+        if(c + 1 < KT_KL) xn[j] = LT ? *(const uint4*)(xal + (ar ^ ((c + 1) * 32)) + 256 * j) : xa[LT ? 0 : 2 * (c + 1) + j];
 #pragma unroll
       for(int j = 0; j < 2; ++j){
         const int s = s_lo + j, u = s * KT_KL + c;
@@ -694,10 +707,10 @@ __global__ void __launch_bounds__(64 * KM_Q8_KS) k_q8_mma(const KtGemvArgs a, co
   }
 }
 
-#define KQ8(GRP, DBG, MS) template __global__ void k_q8_mma<GRP, DBG, MS>(const KtGemvArgs, const KtGroupedArgs, \
-    const int8_t*, const float*, int32_t*, int);
-KQ8(false, false, false) KQ8(false, true, false) KQ8(true, false, false) KQ8(true, true, false)
-KQ8(true, false, true) KQ8(true, true, true)
+#define KQ8(GRP, MS, LT) template __global__ void k_q8_mma<GRP, false, MS, LT>(const KtGemvArgs, const KtGroupedArgs, \
+    const int8_t*, const float*, int32_t*, int); template __global__ void k_q8_mma<GRP, true, MS, LT>(const KtGemvArgs, \
+    const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
+KQ8(false, false, true) KQ8(true, false, true) KQ8(true, false, false) KQ8(true, true, true) KQ8(true, true, false)
 #undef KQ8
 
 #ifdef KT_TRACE

@@ -63,8 +63,8 @@ def _kernels(text):
     return out
 
 
-SCRATCH_OK = {"k_gemv_flat1<0, 1, true, false>", "k_gemv_pair<true>", "k_q8_mma<false, true, false>",
-              "k_q8_mma<true, true, false>", "k_tern_gemm8<true>", "k_gemv_m16<true, 2, true, true>"}
+SCRATCH_OK = {"k_gemv_flat1<0, 1, true, false>", "k_gemv_pair<true>", "k_q8_mma<false, true, false, true>",
+              "k_q8_mma<true, true, false, true>", "k_q8_mma<true, true, false, false>", "k_tern_gemm8<true>", "k_gemv_m16<true, 2, true, true>"}
 
 
 def _demangle(names):

@@ -60,6 +60,20 @@ def test_grouped_passes(C, lens):
     _grouped(100, C, lens)
 
 
+# k_q8_mma's activations straight into the operand and through LDS: 5 and 8 entries an expert over 1 to 8 slices, lists around a
+# pass of 16 and of two passes
+FIVE = [0, 1, 16, 17, 2, 3, 1, 0]
+EIGHT = [0, 1, 16, 17, 30, 2, 1, 0]
+
+
+@gpu
+@pytest.mark.parametrize("lens", [FIVE, EIGHT], ids=["five", "eight"])
+@pytest.mark.parametrize("C", [512, 768, 1856, 2688, 3584, 4096])
+def test_grouped_either_way(C, lens):
+    assert sum(lens) // len(lens) == (5 if lens is FIVE else 8)
+    _grouped(100, C, lens)
+
+
 def _active(cnt):
     """the active experts in ascending order (E entries, the tail unused) and how many there are"""
     on = np.flatnonzero(cnt)
@@ -68,7 +82,7 @@ def _active(cnt):
     return act, np.array([len(on)], np.int32)
 
 
-@pytest.mark.parametrize("lens", [LENS, FEW, LONG3, LONG3B, LONG7])
+@pytest.mark.parametrize("lens", [LENS, FEW, LONG3, LONG3B, LONG7, FIVE, EIGHT])
 def test_lists_are_whole(lens):
     """the lists that the tests here hand to the kernel, which trusts them: every active expert once, none past the table"""
     act, nact = _active(np.array(lens, np.int32))
