@@ -31,7 +31,7 @@ __global__ void k_gemv_m16(const KtGemvArgs, const int8_t*, const float*, const 
 template <bool GRP, bool DBG, bool MS, bool LT>
 __global__ void k_q8_mma(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int);
 template <bool GRP, bool DBG>
-__global__ void k_q8_gemm(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int, int);
+__global__ void k_q8_gemm(const KtGemvArgs, const KtGroupedArgs, const int8_t*, const float*, int32_t*, int, int, int);
 template <int SRC> __global__ void k_tern_pack(const uint8_t*, const uint16_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_q8_pack(const uint8_t*, int, int, uint32_t*, uint16_t*);
 extern "C" __global__ void k_tern_pack_ptq1(const uint8_t*, int, int, int, int, uint32_t*, uint16_t*);
@@ -761,8 +761,8 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
      && (long long)M * ldq < (1ll << 31)
      && (long long)M * ldd * 4 < (1ll << 31) && (long long)kt_r8(R) * NB * 272 < (1ll << 31) && (M + 63) / 64 <= 65535){
     const dim3 grid((R + 127) / 128, (M + 63) / 64);
-    if(dbg) KT_LAUNCH((k_q8_gemm<false, true>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks, 1);
-    else KT_LAUNCH((k_q8_gemm<false, false>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks, 1);
+    if(dbg) KT_LAUNCH((k_q8_gemm<false, true>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks, 1, 1);
+    else KT_LAUNCH((k_q8_gemm<false, false>), grid, dim3(256), 0, kt_stream(stream), a, ga, Q, D, dbg, ks, 1, 1);
     return 0;
   }
   if((M >= 9 || (M >= 5 && nw >= 1ll << 22) || (M >= 3 && nw >= 1ll << 25)) && ks <= KT_Q8_MMA_KS
@@ -846,13 +846,24 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
   const int ks = kt_kslices(a.NU);
   const int ny = E < nentries ? E : nentries;
   hipStream_t s = kt_stream(stream);
-  /* Entries an expert on average from which k_q8_gemm, whose two tiles of 32 entries a wave share the weights, is faster
-     (MI355X, k_q8_mma against it; router scores with a bias of 0.1 N(0, 1), as popular experts have, up [1856 x 2688] / down
-     [2688 x 1856] of 128 experts, 6 picks): 96 entries 1003 / 976 -> 398 / 391 us, 24: 310 / 304 -> 174 / 179, 12: 195 / 182 -> 146 /
-     147, 9: 170 / 152 -> 130 / 133, 7: 146 / 149 -> 131 / 134, but 5: 117 / 120 against 107 / 122 and 4: 109 against 114 down; with no
-     bias 8: 154 against 156, 6: 149 against 153. So 8, where neither router loses; 10 where the rows have up to 2 slices ([1000 x 512] of 64 experts at 8 / 9
-     entries 18.9 / 18.8 against 19.8 / 18.7), 4 where they have more slices than k_q8_mma takes */
-  const long long many = ks <= 2 ? 10 : ks <= KT_Q8_MMA_KS ? 8 : 4;
+  int cus = 0;
+  const int ec = kt_cu_count(&cus);
+  if(ec) return ec;
+  /* Which kernel, by the entries an expert on average, the slices of a row (ks) and k_q8_gemm's blocks (a row tile of 128 of
+     an expert; its two tiles of 32 entries a wave share the weights). MI355X, us, even router / router scores with a bias of 0.25
+     N(0, 1), k_q8_mma against k_q8_gemm:
+     - more than 8 slices: k_q8_gemm from 4 entries ([1024 x 5120] of 32 experts 64 against 41; k_q8_mma does not take them);
+     - up to a block a CU: from 11, since k_q8_mma's grid is four times as large: [1024 x 4096] of 32 experts at 10 28.8 / 44 against 33.8,
+       at 12 46 / 47 against 33.9, [1856 x 2688] of 16 at 8 / 10 / 12 21.4 / 21.9 / 33.4 against 26.4; two slices from 32 ([512 x 1024]
+       of 32 at 13 12.5 / 14.1 against 12.3 / 17.7, at 24 14.8 / 14.7 against 17.2), one from 10 ([512 x 512] of 32 at 10 9.9 against 8.2);
+     - fewer than 24 units (768 columns), more than two blocks a CU: from 20 ([2496 x 544] of 64 experts at 12 37.2 / 39.0 against 40.6;
+       [4096 x 512] of 32 at 12 21.8 / 22.1 against 23.9, at 16 23.6 / 24.0 against 24.3, at 20 25.5 / 27.5 against 24.6);
+     - up to two slices: from 10 ([2048 x 768] of 128 experts at 8 59.0 / 59.9 against 61.4, at 12 60.9 / 64.6 against 61.9);
+     - else from 8 ([1856 x 2688] of 128 experts at 8 141 / 155 against 143.6 / 142, at 9 145 / 161 against 145 / 144, [768 x 2048] at
+       8 48.0 / 54.8 against 48.6) */
+  const long long tiles = (long long)((R + 127) / 128) * ny;
+  const long long many = ks > KT_Q8_MMA_KS ? 4 : tiles <= cus ? (ks == 1 ? 10 : ks == 2 ? 32 : 11) :
+                         a.NU < 3 * KT_KL && tiles > 2ll * cus ? 20 : ks <= 2 ? 10 : 8;
   const bool off32 = (long long)a.nrows * ldq < (1ll << 31) && (long long)a.nrows * ldd * 4 < (1ll << 31)
                      && (long long)kt_r8(R) * a.NU * 272 < (1ll << 31);
   if(nentries >= many * ny && off32 && kt_q8_gemm_takes(a.NU)){
@@ -861,10 +872,16 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
        / 260; without the bias 396 / 385 / 392. Odd: the blocks past a list's end leave at once, and an even P left the same
        half of the shader engines with them (P 2 and 4 at 96 entries: 422 and 745 us) */
     const int P = nentries / ny < 64 ? 3 : 7;
-    const dim3 grid((unsigned)(((long long)((R + 127) / 128) * ny + 7) / 8 * 8 * P));
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8 * P));
+    /* grids of up to two blocks a CU, which are resident at once, and short lists: the blocks with a list's first pass come
+       before the others. Between blocks that leave at once they landed on part of the CUs: [1856 x 2688] of 16 experts at 12 entries
+       34.0 -> 26.4 us, [2048 x 4096] of 32 73.5 -> 54.4, [1000 x 1024] of 64 23.5 -> 17.2, at 20 25.0 -> 17.6. At more entries a popular
+       expert's later passes would wait for those (with a bias of 0.7 N(0, 1) [1024 x 3072] of 64 at 20 61.6 against 79.2, but
+       [1000 x 1024] 30.6 against 31.8: short rows up to 32 entries) */
+    const int dv = tiles <= 2ll * cus && nentries < (ks <= 2 ? 32ll : 16ll) * ny ? -(int)((tiles + 7) / 8) : P;
     const KtGemvArgs da = {};
-    if(dbg) KT_LAUNCH((k_q8_gemm<true, true>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P);
-    else KT_LAUNCH((k_q8_gemm<true, false>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P);
+    if(dbg) KT_LAUNCH((k_q8_gemm<true, true>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P, dv);
+    else KT_LAUNCH((k_q8_gemm<true, false>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P, dv);
     return 0;
   }
   /* the matrix-core kernel reads the input rows through a buffer resource with 32-bit offsets */

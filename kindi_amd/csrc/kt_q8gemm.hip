@@ -17,8 +17,8 @@
 
    Measured on MI355X (128 experts, 6 picks, even router, up [1856 x 2688] / down [2688 x 1856], against k_q8_mma): 96
    entries an expert 1003 / 981 -> 394 / 372 us, 24: 309 / 302 -> 174 / 157, 12: 166 / 168 -> 152 / 151 (678 MB of weights: 4.5 TB/s).
-   The refill after a block's last slice reads an empty buffer: with the first slice read again there (KS + 1 slices for KS) 12
-   entries took 156 / 167 us, 24: 178 / 176. At long lists the SIMDs bound it: a unit of a tile takes
+   Nothing is refilled after a block's last slice: with the first slice read again there (KS + 1 slices for KS) 12 entries took
+   156 / 167 us, 24: 178 / 176; from an empty buffer instead of behind a branch every length is 1 to 2% slower. At long lists the SIMDs bound it: a unit of a tile takes
    about 37 vector and 1.5 matrix instructions, and 2 waves a SIMD (253 registers) issue at most one vector instruction
    each about every 4 cycles; without any global load 96 entries take 296 us. */
 #include <type_traits>
@@ -55,7 +55,7 @@ __device__ __forceinline__ void qg_ldw(const __amdgpu_buffer_rsrc_t rw, int c, i
 
 template <bool GRP, bool DBG>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 1 : 2))) k_q8_gemm(const KtGemvArgs a,
-    const KtGroupedArgs ga, const int8_t* __restrict__ xq, const float* __restrict__ xd, int32_t* __restrict__ dbg, int KS, int P){
+    const KtGroupedArgs ga, const int8_t* __restrict__ xq, const float* __restrict__ xd, int32_t* __restrict__ dbg, int KS, int P, int dv){
   __shared__ __attribute__((aligned(16))) KtQg L;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, n = lane & 31;
@@ -64,10 +64,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
   int R, NU, ldy, ldq, ldd, nrows, t_lo, t_hi, t_st, p0 = 0, bx;
   const int* xrow = nullptr;
   if(GRP){
-    /* blocks of one row tile, P of them (passes z, z + P, ..), 8 ids apart: on one XCD at one time, so that its L2 serves
-       the weights to all but the first */
-    const int gx = (ga.R + 127) >> 7, z = (int)(blockIdx.x >> 3) % P;
-    const int tile = ((int)(blockIdx.x >> 3) / P) * 8 + (int)(blockIdx.x & 7), ie = tile / gx;
+    /* P blocks of one row tile (passes z, z + P, ..) on one XCD, so that its L2 serves the weights to all but the first. dv = P: 8
+       ids apart, at one time. dv < 0 (minus the row tiles an XCD): the tiles' first passes before all others */
+    const unsigned gx = (unsigned)(ga.R + 127) >> 7, q = blockIdx.x >> 3, dq = q / (unsigned)abs(dv), dr = q - dq * (unsigned)abs(dv);
+    const int z = dv > 0 ? dr : dq;
+    const unsigned tile = (dv > 0 ? dq : dr) * 8 + (blockIdx.x & 7);
+    const int ie = tile / gx;
     bx = tile - ie * gx;
     const int nact = *ga.nact;
     if(ie >= nact) return;
@@ -86,7 +88,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
   const uint32_t OOB = 0x80000000u;
   const kt_v4i rx = kt_dma_rsrc(xq, (uint32_t)nrows * (uint32_t)ldq);
   const kt_v4i rs = kt_dma_rsrc(xd, (uint32_t)nrows * (uint32_t)ldd * 4u);
-  __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)wbuf, (short)0, R8 * NU * 272, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)wbuf, (short)0, R8 * NU * 272, 0x00020000);
   const uint32_t la = kt_dma_lds(L.a), lx = kt_dma_lds(L.x);
   const int ao = n * 512 + ((h ^ (n & 15)) << 4), xo = n * 64 + ((2 * h) ^ ((n >> 2) & 3)) * 16;   /* this lane's operands */
   const uint32_t wb = rg < R8 ? (uint32_t)(rg * NU * 16 + (row & 7)) * 16u : OOB;
@@ -211,9 +213,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
         refilled = tt + 1 == T;
         if(!refilled) issue(st ^ 1, tt + 1, s0, ns);
         else if(k + 1 < KS) issue(st ^ 1, 0, sn, nsn);
-        /* the refill after the block's last slice has nothing to fetch: an empty buffer's loads make no memory access */
-        if(k + 1 == KS && t0 + t_st >= t_hi) rw = __builtin_amdgcn_make_buffer_rsrc((void*)wbuf, (short)0, 0, 0x00020000);
-        tile(refilled, st, tt, k, s0, ns, sn, nsn, t0);
+        tile(refilled && (k + 1 < KS || t0 + t_st < t_hi), st, tt, k, s0, ns, sn, nsn, t0);
         st ^= 1;
       }
     }
@@ -222,5 +222,5 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DBG ? 
 }
 
 #define KT_QG(GRP, DBG) template __global__ void k_q8_gemm<GRP, DBG>(const KtGemvArgs, const KtGroupedArgs, const int8_t*, \
-    const float*, int32_t*, int, int);
+    const float*, int32_t*, int, int, int);
 KT_QG(false, false) KT_QG(false, true) KT_QG(true, false) KT_QG(true, true)

@@ -74,6 +74,18 @@ def test_grouped_either_way(C, lens):
     _grouped(100, C, lens)
 
 
+# few entries an expert on a small grid: the blocks with the lists' first passes before all others (a second pass of the first
+# ones at 200 entries), numbers of row tiles that are no multiple of 8, an idle expert last
+FIRST = [200, 0, 70, 33, 1] + [0] * 8 + [2, 1, 64, 0, 0, 0, 0, 7, 0, 0, 0, 5, 0]
+
+
+@gpu
+@pytest.mark.parametrize("R,C", [(100, 512), (129, 1856), (300, 2688), (129, 4352)])
+def test_grouped_first_passes_first(R, C):
+    assert 11 * len(FIRST) <= sum(FIRST) < 16 * len(FIRST) and max(FIRST) > 192
+    _grouped(R, C, FIRST)
+
+
 def _active(cnt):
     """the active experts in ascending order (E entries, the tail unused) and how many there are"""
     on = np.flatnonzero(cnt)
@@ -82,7 +94,7 @@ def _active(cnt):
     return act, np.array([len(on)], np.int32)
 
 
-@pytest.mark.parametrize("lens", [LENS, FEW, LONG3, LONG3B, LONG7, FIVE, EIGHT])
+@pytest.mark.parametrize("lens", [LENS, FEW, LONG3, LONG3B, LONG7, FIVE, EIGHT, FIRST])
 def test_lists_are_whole(lens):
     """the lists that the tests here hand to the kernel, which trusts them: every active expert once, none past the table"""
     act, nact = _active(np.array(lens, np.int32))
