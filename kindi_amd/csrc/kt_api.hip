@@ -739,9 +739,10 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
      - the matrix cores with a K slice a wave (k_q8_mma, up to 8 slices) from 9 tokens, from 5 on 2^22 weights, from 3 on
        2^25: [2688 x 1856] at 4 / 5 tokens 6.4 against 7.4 / 8.3 -> 7.3 us, [8192 x 4096] at 3 tokens 14.2 -> 11.5,
        [1024 x 1024] at 5 / 10 tokens 6.1 against 6.8 / 8.1 -> 6.9;
-     - k_q8_gemm (above 16 tokens) above ks + 4 (tile of 32 rows, pass of 16 tokens) pairs a CU, 3 where a row is one slice. k_q8_gemm's time
-       goes with the steps of a row, k_q8_mma's with the pairs and little with the slices. Pairs, us on k_q8_mma / k_q8_gemm: ks 1
-       [8192 x 512] 3 11.0 / 10.3, 4 13.7 / 10.4; ks 2 [8192 x 1024] 4 15.2 / 16.6, 7 23.4 / 17.0, [16384 x 1024] 6 14.3 / 16.8; ks 3 [8192 x
+     - k_q8_gemm (above 16 tokens) where a k_q8_mma block has more than ks + 4 passes of 16 tokens, times its tiles a CU above one; 3
+       where a row is one slice ([6753 x 1632] at 168 tokens, 6 passes in two blocks a tile, 25.4 / 29.2, [7365 x 1696] at 242, 8, 34.7 / 30.4). k_q8_gemm's time
+       goes with the steps of a row, k_q8_mma's with the pairs and little with the slices. Passes, us on k_q8_mma / k_q8_gemm: ks 1
+       [8192 x 512] 3 11.0 / 10.3, 4 13.7 / 10.4; ks 2 [8192 x 1024] 4 15.2 / 16.6, 7 23.4 / 17.0, [16384 x 1024] 2 x 3 14.3 / 16.8; ks 3 [8192 x
        1536] 5 19.1 / 23.1, 8 27.6 / 23.7; ks 4 [8192 x 2048] 7 25.8 / 28.9, 9 31.7 / 29.1; ks 5 [8192 x 2560] 9 34.4 / 35.4, 10 37.4 /
        35.1; ks 6 [8192 x 2688] 10 37.8 / 40.9, 11 41.2 / 40.8; ks 8 [8192 x 4096] 11 49 / 56, 14 59 / 56;
      - above 8 slices k_q8_gemm against the v_dot4 kernel, whose time goes with tokens times its rounds of row groups over the
@@ -755,8 +756,14 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
   if(ec) return ec;
   const int tiles = (kt_r8(R) + 3) / 4, np = M / 16 + (M % 16 ? 1 : 0);
   const long long nw = (long long)R * C;
+  /* k_q8_mma's blocks a tile, its passes dealt over them: as many as give each CU one block. Up to 4 slices two blocks (of ks
+     waves, 256 registers a lane) share a CU, so some CUs may get a second one; wider blocks would wait for a second round:
+     [8145 x 3392] (255 tiles) at 18 tokens in two blocks a tile 19.1 us, in one 14.0, [5919 x 2528] at 34 18.1, 14.7 */
+  const int want = ks <= 4 ? (cus + tiles - 1) / tiles : cus / tiles > 1 ? cus / tiles : 1, gy = want < np ? want : np;
+  /* a block's passes, times CUs; a fifth more where blocks of one tile share CUs */
+  const long long load = (long long)((np + gy - 1) / gy) * (tiles > cus ? tiles : cus) * (gy > 1 && tiles * gy > cus ? 6 : 5);
   const int rounds = (kt_r8(R) + cus - 1) / cus;
-  if((ks <= KT_Q8_MMA_KS ? M > 16 && (long long)tiles * np > (ks == 1 ? 3ll : ks + 4ll) * cus
+  if((ks <= KT_Q8_MMA_KS ? M > 16 && load > 5 * (ks == 1 ? 3ll : ks + 4ll) * cus
                          : M >= 9 && (long long)M * rounds >= (M > 32 ? 88 : 50)) && kt_q8_gemm_takes(NB)
      && (long long)M * ldq < (1ll << 31)
      && (long long)M * ldd * 4 < (1ll << 31) && (long long)kt_r8(R) * NB * 272 < (1ll << 31) && (M + 63) / 64 <= 65535){
@@ -767,9 +774,8 @@ int kt_q8_gemv(const void* W, int R, int C, const int8_t* Q, int ldq, const floa
   }
   if((M >= 9 || (M >= 5 && nw >= 1ll << 22) || (M >= 3 && nw >= 1ll << 25)) && ks <= KT_Q8_MMA_KS
      && (long long)M * ldq < (1ll << 31)){
-    /* tiles of 32 rows, the passes of 16 tokens dealt over as many blocks as give each CU one (of ks waves, 256 registers a
-       lane): [4096 x 2688] at 50 tokens 18.7 -> 12.6 us, [1024 x 1024] at 128 25.4 -> 7.5; two a CU was no faster */
-    const int want = (cus + tiles - 1) / tiles, gy = want < np ? want : np;
+    /* tiles of 32 rows, passes of 16 tokens: [4096 x 2688] at 50 tokens in one block a tile 18.7 us, in two 12.6, [1024 x 1024] at 128
+       25.4, in 8 7.5 */
     const dim3 grid(tiles, gy), block(64 * ks);
     const size_t lds = (size_t)ks * (16 * 32 * 4 + 256 * 4) + (size_t)ks * KT_Q8_MMA_ACT;   /* slice sums, D, activations */
     if(dbg) KT_LAUNCH((k_q8_mma<false, true, false, true>), grid, block, lds, kt_stream(stream), a, ga, Q, D, dbg, ks);

@@ -137,7 +137,8 @@ def _grouped(R, C, lens):
 @gpu
 @pytest.mark.parametrize("R,C,M", [(8, 32, 3), (100, 96, 9), (2688, 1856, 5), (4096, 2688, 50), (4100, 2688, 330),
                                    (8192, 4096, 4), (8190, 1024, 161), (4100, 2688, 400), (8190, 1024, 200), (130, 4352, 64), (136, 16384, 65), (136, 8192, 65), (40, 8192, 70),
-                                   (8190, 512, 48), (8190, 512, 49), (8190, 1024, 96), (8190, 1024, 97), (136, 4352, 88), (4100, 4352, 16), (4100, 4352, 17), (4090, 4352, 25), (4090, 4352, 43), (4090, 4352, 44)])
+                                   (8190, 512, 48), (8190, 512, 49), (8190, 1024, 96), (8190, 1024, 97), (136, 4352, 88), (4100, 4352, 16), (4100, 4352, 17), (4090, 4352, 25), (4090, 4352, 43), (4090, 4352, 44),
+                                   (5919, 2528, 34), (4130, 1632, 49), (7365, 1696, 242)])
 def test_dense_routes(R, C, M):
     from kindi_amd import moe
     say("q8 dense", R, C, M)
