@@ -215,9 +215,9 @@ __global__ void __launch_bounds__(512) k_fold_q8(const KtFoldArgs a){
    where their addresses allow (vec). rmsfold: one block a row; the norm's sum is taken first in the reference's order
    (thread j over columns j + 512 m), the row kept in LDS.
    MI355X, 1000 tokens, against the kernel above on chunks of up to 8192 columns (rmsfold: the row): smfold of 12288 columns, HB
-   4096, 45.1 -> 30.3 us, rmsfold of 4096 with one part and xw 21.3 -> 15.1, of 5120 at 33 / 256 tokens 10.2 / 11.3 -> 7.0 / 8.0.
-   waves_per_eu holds the registers to three blocks a CU for rmsfold (80; 88 and two blocks without: 57.8 against 66.5 us at
-   4096 tokens of 8192 columns) and to five waves a SIMD for smfold (3 %). */
+   4096, 45.1 -> 29.0 us, rmsfold of 4096 with one part and xw 21.3 -> 15.1, of 5120 at 33 / 256 tokens 10.2 / 11.3 -> 7.0 / 8.0.
+   waves_per_eu holds the registers to three blocks a CU (80): rmsfold 57.8 against 66.5 us at 4096 tokens of 8192 columns (88 and
+   two blocks without), smfold 51.3 against 56.5 at 2048 of 12288 (82 and two), 9.6 against 10.9 at 2048 of 1024 in HB 512. */
 #define KF_VX 1                       /* x / r rows, sg and w in 16-byte loads */
 #define KF_VO 2                       /* xw, xn, xo in 16-byte stores */
 #define KF_VQ 4                       /* the int8 rows in 8-byte stores */
@@ -233,7 +233,7 @@ __device__ __forceinline__ void kf_ld8(float* v, const float* p, bool vec){
 /* a wave's 512 columns (lane l: 8 l .. + 7) to p, through t, 512 floats of LDS of the wave's own, so that a store's lanes are
    neighbours. Straight from the lanes a 16-byte store leaves every other 16 bytes of its lines to the next one: MI355X,
    rmsfold of 4096 columns with xw, xn and xo at 1000 / 4096 tokens 37.5 / 142 us that way, 18.6 / 70 so; smfold of 12288 with
-   xo 50.4 / 212 against 32.9 / 148. kf_out: columns that t already holds */
+   xo 50.4 / 212 against 32.9 / 148 (at two blocks a CU). kf_out: columns that t already holds */
 __device__ __forceinline__ void kf_put8(float* t, const float* v, int l){
   *(float4*)(t + 8 * l) = make_float4(v[0], v[1], v[2], v[3]);
   *(float4*)(t + 8 * l + 4) = make_float4(v[4], v[5], v[6], v[7]);
@@ -265,7 +265,7 @@ __device__ __forceinline__ void kf_stq(int8_t* p, const int* q, bool vec){
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE == 0 ? 6 : MODE == 2 ? 5 : 2))) k_fold_many(const KtFoldArgs a, int vec){
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE == 1 ? 2 : 6))) k_fold_many(const KtFoldArgs a, int vec){
   extern __shared__ __attribute__((aligned(16))) float kf_lds[];    /* [8][2][64][4] exchange (2 KB a wave), then the row */
   __shared__ double red[16];
   float4* ex = (float4*)kf_lds;
@@ -303,8 +303,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE =
     }
     s = kf_norm(acc, red, j, C);                                   /* its barrier covers the row too */
   }
-  /* smfold's product for columns c .. c + 7 */
-  auto silu = [&](int c, float* f){
+  /* smfold's product for columns c .. c + 7; ld: loads to issue before its own, but behind single ones (registers) */
+  auto silu = [&](int c, float* f, auto&& ld){
     const float* pa = a.x + (long long)n * a.ldx;
     const float* pb = a.r + (long long)n * a.ldr;
     float fb[8];
@@ -312,12 +312,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE =
       auto src = [&](int e){ const int h = e % a.hd, g = e / a.hd; return h + a.hd * (g / a.rep + a.nk * (g % a.rep)); };
       if(a.hd % 8 == 0){                                           /* uniform: the 8 columns stay neighbours */
         const int sc = src(c);
+        ld();
         kf_ld8(f, pa + sc, vx);
         kf_ld8(fb, pb + sc, vx);
-      } else
+      } else {
 #pragma unroll
         for(int i = 0; i < 8; ++i){ const int sc = src(c + i); f[i] = pa[sc]; fb[i] = pb[sc]; }
-    } else { kf_ld8(f, pa + c, vx); kf_ld8(fb, pb + c, vx); }
+        ld();
+      }
+    } else { ld(); kf_ld8(f, pa + c, vx); kf_ld8(fb, pb + c, vx); }
 #pragma unroll
     for(int i = 0; i < 8; ++i) f[i] = (f[i] / (1.0f + expf(-f[i]))) * fb[i];
   };
@@ -325,7 +328,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE =
   if(MODE == 2 && whole){
     for(int c = 512 * w + 8 * l; c < C; c += 4096){
       float f[8];
-      silu(c, f);
+      silu(c, f, []{});
       kf_put8(rowb + c - 8 * l, f, l);
     }
     __syncthreads();
@@ -342,7 +345,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE =
         kt_wave_sync();
       }
       float sg[8];
-      kf_ld8(sg, a.sg + c, vx);
+      auto ld_sg = [&]{ kf_ld8(sg, a.sg + c, vx); };
+      if(MODE != 2 || whole) ld_sg();
       if(MODE == 0){
         float f[8], wv[8];
         kf_ld8(f, rowb + c, true);
@@ -360,7 +364,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MODE =
       } else {
         float f[8];
         if(whole) kf_ld8(f, rowb + c, true);
-        else silu(c, f);
+        else silu(c, f, ld_sg);
 #pragma unroll
         for(int i = 0; i < 8; ++i) v[i] = sg[i] * f[i];
       }
@@ -456,7 +460,7 @@ template __global__ void k_fold_many<2>(const KtFoldArgs, int);
 /* ... and rows of up to KF_NARROW columns at any number of tokens, where k_fold_many would leave 6 or 7 of a block's 8 waves
    without columns of their own (MI355X, 64 / 4096 tokens, k_fold_many against k_fold_q8: rmsfold of 512 columns with one part
    4.3 / 19.6 -> 3.6 / 15.0 us, of 1024 in HB 1024 4.8 / 26.5 -> 4.2 / 21.7, smfold 3.6 / 13.7 -> 3.1 / 10.9 and 4.1 / 23.7 -> 3.8 /
-   18.1). Not fold (512: 3.0 / 9.8 us on k_fold_q8, 2.9 / 5.5 on k_fold_many), nor smfold of two HB blocks (18.3 against 17.0) */
+   18.1). Not fold (512: 3.0 / 9.8 us on k_fold_q8, 2.9 / 5.5 on k_fold_many), nor smfold of two HB blocks (18.3 against 16.1) */
 #define KF_NARROW 1024
 #define KF_ROW_MAX 36352              /* columns of a row in LDS beside the exchange (160 KB a CU) */
 
