@@ -190,3 +190,15 @@ def test_moe_and_producer_records(kt, M):
     assert n == 1
     replay_raw(gpudrv, recs, n)
     assert np.array_equal(host(out.XQ), q1) and np.array_equal(host(out.XS), s1) and np.array_equal(host(out.XA), x1)
+
+
+def test_stream_handle_without_the_private_getter(monkeypatch):
+    """the current stream's handle by torch's public interface is the same one (where the raw getter is missing)"""
+    from kindi_amd import linear
+    s = torch.cuda.Stream()
+    for cur in (torch.cuda.current_stream(), s):
+        with torch.cuda.stream(cur):
+            a = linear.stream().value
+            with monkeypatch.context() as m:
+                m.setattr(linear, "_RAW", None)
+                assert linear.stream().value == a == (cur.cuda_stream or None)
