@@ -668,8 +668,12 @@ int kt_tern_gemm8(const int8_t* W8, const void* W, int R, int C, const int8_t* X
   if(ec) return ec;
   const bool aligned = ldy % 8 == 0 && (!Y || kt_al(Y, 16)) && (!Y16 || kt_al(Y16, 16));   /* 16-byte output rows */
 #ifndef KT_G8_MIN_PCT
-#define KT_G8_MIN_PCT 70              /* tiles a CU, percent (measured on MI355X: gate/up [12288 x 4096] at 512 tokens,
-                                         192 tiles on 256 CUs, 46 us on the packed trits, 41.9 here) */
+#define KT_G8_MIN_PCT 70              /* tiles a CU, percent. MI355X, us on the packed trits / here, tiles a CU in brackets: [12288 x
+                                         4096] at 512 tokens (0.75) 41.3 / 37.6, [6144 x 2048] at 1024 (0.75) 24.1 / 21.7, [4096 x 4096] at
+                                         1536 (0.75) 42.6 / 37.5, [17408 x 5120] at 384 (0.80) 54 / 48, [4096 x 12288] at 2048 (1) 130 / 111,
+                                         [12288 x 4096] at 2048 (3) 131 / 118; not where the last round of tiles is short: [17408 x 5120] at
+                                         512 (1.06) 68 / 89, [12288 x 4096] at 768 (1.12) 60 / 72, at 1536 (2.25) 100 / 109, [5120 x 17408] at
+                                         2048 (1.25) 220 / 279 */
 #endif
   if((long long)((kt_r8(R) * KT_RG + 255) / 256) * ((M + 127) / 128) * 100 < (long long)cus * KT_G8_MIN_PCT || !aligned)
     return kt_tern_gemm(W, R, C, XQ, ldq, XS, nullptr, 1, M, Y, Y16, ldy, dbg, stream);

@@ -15,7 +15,7 @@
    V_MFMA_F32_32X32X1 (an outer product: one rounding, as the multiply), so that the token scales are one LDS word a lane
    and not a broadcast of 16.
 
-   What bounds it: a SIMD runs its matrix and vector instructions one after the other (a register-only probe: 4 MFMAs
+   What bounds it: a SIMD overlaps its matrix and vector instructions little (a register-only probe: 4 MFMAs
    69 ns, with 32 vector operations 92, with 64 128, with 128 203), so a tile's group costs 70 ns of MFMA and about 1 ns a
    vector operation: 32 of the epilogue, 44 / T of the unpacking; the LDS reads of the activations (4 KB a tile) come on
    top. Four tiles a wave take 11 operations of unpacking instead of 22, but two waves a SIMD and measured no better.

@@ -21,8 +21,9 @@
    overlaps an MFMA only when it sits behind it in the stream). One block a CU (its 145 KB of LDS) takes tiles
    blockIdx.x, + gridDim.x, ...; a tile's outputs go out through LDS as 16-byte token rows before the next tile's
    first DMAs.
-   Measured on MI355X (config 2, M = 2048, fp16 out): gate/up [12288 x 4096] 118 .. 131 us against 138 for k_tern_gemm_w on the
-   packed trits, down [4096 x 12288] 118 .. 128 us (with two-byte stores straight from the accumulators: 175 and 142 us).
+   Measured on MI355X (M = 2048, fp16 out, back-to-back graphs, against k_tern_gemm_w on the packed trits): gate/up [12288 x 4096] 118
+   against 131 us, down [4096 x 12288] 111 against 130, [4096 x 4096] 42 against 52; timed alone in a bench run gate/up 153 against 147, down
+   122 against 141 (with two-byte stores straight from the accumulators: gate/up 175, down 142).
    Below 0.7 tiles a CU kt_tern_gemm8 runs the packed-trit kernels. */
 #include "kt_common.h"
 #include "kt_dma.h"

@@ -16,11 +16,11 @@
    A unit past the matrix or the slice gets zero scales (its product is +0).
 
    Measured on MI355X (128 experts, 6 picks, even router, up [1856 x 2688] / down [2688 x 1856], against k_q8_mma): 96
-   entries an expert 1003 / 981 -> 394 / 372 us, 24: 309 / 302 -> 174 / 157, 12: 166 / 168 -> 152 / 151 (678 MB of weights: 4.5 TB/s).
+   entries an expert 987 / 970 -> 386 / 373 us, 20: 271 / 264 -> 149 / 148, 12: 165 / 168 -> 146 / 146 (678 MB of weights: 4.6 TB/s).
    Nothing is refilled after a block's last slice: with the first slice read again there (KS + 1 slices for KS) 12 entries took
-   156 / 167 us, 24: 178 / 176; from an empty buffer instead of behind a branch every length is 1 to 2% slower. At long lists the SIMDs bound it: a unit of a tile takes
-   about 37 vector and 1.5 matrix instructions, and 2 waves a SIMD (253 registers) issue at most one vector instruction
-   each about every 4 cycles; without any global load 96 entries take 296 us. */
+   156 / 167 us, 24: 178 / 176; from an empty buffer instead of behind a branch every length is 1 to 2% slower. At long
+   lists (96 entries) counters give vector instructions 53% of the SIMDs' cycles and the matrix cores 17%, next to no overlap (a unit's
+   results are taken at once), the rest waiting with 2 waves a SIMD (253 registers); without any global load they take 296 us. */
 #include <type_traits>
 #include "kt_common.h"
 #include "kt_dma.h"
