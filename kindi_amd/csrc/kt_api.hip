@@ -863,7 +863,8 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
      an expert; its two tiles of 32 entries a wave share the weights). MI355X, us, even router / router scores with a bias of 0.25
      N(0, 1), k_q8_mma against k_q8_gemm:
      - more than 8 slices: k_q8_gemm from 4 entries ([1024 x 5120] of 32 experts 64 against 41; k_q8_mma does not take them);
-     - up to a block a CU: from 11, since k_q8_mma's grid is four times as large: [1024 x 4096] of 32 experts at 10 28.8 / 44 against 33.8,
+     - up to a block a CU: from 11, 12 and 13 by the number of lists (the longest of few lists keeps to one pass of k_q8_mma longer:
+       [1480 x 2944] of 8 at 12 17.8 against 25.3), since k_q8_mma's grid is four times as large: [1024 x 4096] of 32 experts at 10 28.8 / 44 against 33.8,
        at 12 46 / 47 against 33.9, [1856 x 2688] of 16 at 8 / 10 / 12 21.4 / 21.9 / 33.4 against 26.4; two slices from 32 ([512 x 1024]
        of 32 at 13 12.5 / 14.1 against 12.3 / 17.7, at 24 14.8 / 14.7 against 17.2), one from 10 ([512 x 512] of 32 at 10 9.9 against 8.2);
      - fewer than 24 units (768 columns), more than two blocks a CU: from 20 ([2496 x 544] of 64 experts at 12 37.2 / 39.0 against 40.6;
@@ -872,7 +873,7 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
      - else from 8 ([1856 x 2688] of 128 experts at 8 141 / 155 against 143.6 / 142, at 9 145 / 161 against 145 / 144, [768 x 2048] at
        8 48.0 / 54.8 against 48.6) */
   const long long tiles = (long long)((R + 127) / 128) * ny;
-  const long long many = ks > KT_Q8_MMA_KS ? 4 : tiles <= cus ? (ks == 1 ? 10 : ks == 2 ? 32 : 11) :
+  const long long many = ks > KT_Q8_MMA_KS ? 4 : tiles <= cus ? (ks == 1 ? 10 : ks == 2 ? 32 : ny <= 8 ? 13 : ny <= 16 ? 12 : 11) :
                          a.NU < 3 * KT_KL && tiles > 2ll * cus ? 20 : ks <= 2 ? 10 : 8;
   const bool off32 = (long long)a.nrows * ldq < (1ll << 31) && (long long)a.nrows * ldd * 4 < (1ll << 31)
                      && (long long)kt_r8(R) * a.NU * 272 < (1ll << 31);
@@ -883,12 +884,12 @@ int kt_q8_grouped(const void* const* Wexp, int R, int C, int E, const int* cnt, 
        half of the shader engines with them (P 2 and 4 at 96 entries: 422 and 745 us) */
     const int P = nentries / ny < 64 ? 3 : 7;
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8 * P));
-    /* grids of up to two blocks a CU, which are resident at once, and short lists: the blocks with a list's first pass come
-       before the others. Between blocks that leave at once they landed on part of the CUs: [1856 x 2688] of 16 experts at 12 entries
-       34.0 -> 26.4 us, [2048 x 4096] of 32 73.5 -> 54.4, [1000 x 1024] of 64 23.5 -> 17.2, at 20 25.0 -> 17.6. At more entries a popular
-       expert's later passes would wait for those (with a bias of 0.7 N(0, 1) [1024 x 3072] of 64 at 20 61.6 against 79.2, but
-       [1000 x 1024] 30.6 against 31.8: short rows up to 32 entries) */
-    const int dv = tiles <= 2ll * cus && nentries < (ks <= 2 ? 32ll : 16ll) * ny ? -(int)((tiles + 7) / 8) : P;
+    /* grids of up to four blocks a CU (two rounds) and short lists: the blocks with a list's first pass come before the others.
+       Between blocks that leave at once they landed on part of the CUs: [1856 x 2688] of 16 experts at 12 entries 34.0 -> 26.4 us, [2048 x
+       4096] of 32 73.5 -> 54.4, [1000 x 1024] of 64 23.5 -> 17.2, at 20 25.0 -> 17.6, [768 x 2048] of 128 at 10 49.4 -> 43.7 (six a CU 3%).
+       At more entries a popular expert's later passes would wait for those (with a bias of 0.7 N(0, 1) [1024 x 3072] of 64 at 20 61.6
+       against 79.2, but [1000 x 1024] 30.6 against 31.8: short rows up to 32 entries) */
+    const int dv = tiles <= 4ll * cus && nentries < (ks <= 2 ? 32ll : 16ll) * ny ? -(int)((tiles + 7) / 8) : P;
     const KtGemvArgs da = {};
     if(dbg) KT_LAUNCH((k_q8_gemm<true, true>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P, dv);
     else KT_LAUNCH((k_q8_gemm<true, false>), grid, dim3(256), 0, s, da, a, Q, D, dbg, ks, P, dv);
